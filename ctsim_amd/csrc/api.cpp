@@ -888,6 +888,7 @@ struct ctsim_batch2 {
     std::vector<void*> d_views;
     int proj_split = 1;  // waves per forward work item (strip split)
     int back_split = 4;  // waves per backprojection work item (view split)
+    int form[2] = {0, 0};  // forward form of DD and SF: 0 candidates, 1 line walk (flat), 2 line walk (arc)
 };
 
 namespace {
@@ -938,6 +939,15 @@ int batch2_build(ctsim_batch2* b, int n, const ctsim_geom* geoms, const int32_t*
     }
     b->nitems_proj = ip;
     b->nitems_back = ib;
+    if constexpr (sizeof(T) == 4) {
+        // the line walk where it covers every slice and the detectors are all of one type
+        for (int kind = 0; kind < 2; ++kind) {
+            bool ok = true;
+            for (int i = 0; i < n; ++i)
+                ok = ok && fan_walk_ok(sl[i].g, kind) && (sl[i].g.dettype == 1) == (sl[0].g.dettype == 1);
+            b->form[kind] = ok ? (sl[0].g.dettype == 1 ? 1 : 2) : 0;
+        }
+    }
     b->proj_split = ip < kFewItems2D ? 4 : 1;  // the single-slice forward's rule
     b->img_elems = img;
     b->sino_elems = sino;
@@ -994,9 +1004,10 @@ int ctsim_batch2_proj(const ctsim_batch2* b, const char* op, const void* d_img, 
     const int kind = k == OP_PROJ_DD ? 0 : 1;
     hipError_t e = b->compute == CTSIM_F32
                        ? fbct_proj_batch_launch<float>(b->d_slices_proj, b->nslices, b->nitems_proj, d_img, img_dt,
-                                                       d_sino, sino_dt, kind, b->proj_split, (hipStream_t)stream)
+                                                       d_sino, sino_dt, kind, b->proj_split, b->form[kind],
+                                                       (hipStream_t)stream)
                        : fbct_proj_batch_launch<double>(b->d_slices_proj, b->nslices, b->nitems_proj, d_img, img_dt,
-                                                        d_sino, sino_dt, kind, b->proj_split, (hipStream_t)stream);
+                                                        d_sino, sino_dt, kind, b->proj_split, 0, (hipStream_t)stream);
     if (e == hipErrorInvalidValue) return fail(CTSIM_EUNSUP, "Error: dtype combination not supported.");
     HIP_TRY(e, "batched forward projection");
     return CTSIM_OK;

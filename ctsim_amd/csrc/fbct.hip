@@ -8,6 +8,10 @@
 // Batched forms take a table of independent slices, each with its own geometry,
 // and walk a flat work list of (slice, view, tile) or (slice, pixel block) items,
 // so slices of uneven size share one launch.
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
 #include "internal.h"
 
 namespace ctsim {
@@ -20,7 +24,268 @@ constexpr int kLineBatch = 12;
 enum Foot2 { F2_DD = 0, F2_TF = 1 };
 
 // ---------------------------------------------------------------------------------
-// forward: one wavefront per (view, 64 detector cells); lanes own cells.  Candidate
+// forward, line walk (FP32): one wavefront per (view, 64 detector cells); lanes own cells.
+// Along an image line (a row where |Y| >= |X| for the ray from the source, else a column)
+// the pixels' footprints meet edge to edge on the detector: the pixel spans the projections
+// of its two minor edges, and edge j is shared by pixels j - 1 and j.  So a cell inverts the
+// line once, to the pixel ja that holds its first boundary, and sums
+//     q_{K-1} + sum_{0 < k < K} c_k (q_{k-1} - q_k),   q = amp * pixel of ja + k,
+// where c_k is the part of the cell before edge ja + k (0 at k = 0 and 1 at k = K, which K
+// guarantees): sum_k (c_{k+1} - c_k) q_k telescoped, the same products of overlap, amplitude
+// and pixel as the pixel-by-pixel footprints.  The edge is measured from the cell's own
+// boundary, u_edge - u_cell = sdd/du a dx (j - xi) / d (a: the ray's major direction cosine,
+// xi: where the boundary crosses the line, in pixel edges), so nothing cancels.  On an arc
+// the same difference is sdd/du atan z with z = (t - k d) / (d + k t) of the order of one
+// cell, where z - z^3 / 3 is exact in FP32.  An SF edge is soft: its two corners (the line's
+// two sides) bound a ramp, and c_k is one minus the ramp's integral over the cell; with
+// |X| dy <= |Y| dx the left pair of a pixel's corners lies before its right pair, as in the
+// sorted trapezoid.
+// amp = dx / max(|cos|, |sin|) / 10 = dx hypot(X, Y) / max(|X|, |Y|) / 10 with (X, Y) the
+// pixel relative to the source.
+//
+// Each wave stages kFanWords words of amp * pixel at a time (16 lines of 100 pixels, or 8 of
+// 196) in LDS, zero outside the image: amp is formed once per pixel, and image columns are
+// read 8 or 16 neighbours at a time instead of one word per image row.  Tiles whose rays
+// straddle |X| = |Y| take both walks, each with the other walk's pixels at zero.
+// fan_walk_ok (host) says which geometries the walk covers; the rest take the candidate form.
+//
+// Issue-bound: 47 vector instructions per (line, 64 cells) all told, against some 230 per 64
+// pixels of the candidate form below with its LDS min / max.  256^2, 360 views, 512 bins, DD:
+// 239 -> 86 us; 64 uneven FP16 slices: 18.4 -> 6.1 ms.  The distance from 64-bit results went
+// from 3.3e-6 to 2.0e-6 (no subtraction of large detector coordinates).
+// ---------------------------------------------------------------------------------
+constexpr int kFanWaves = 6;     // waves per SIMD the line-walk kernels are compiled for
+constexpr int kFanWords = 1600;  // staged words per wave: six 4-wave blocks fit a CU's LDS
+
+struct FanLane {          // one walk, per lane (cell) unless noted
+    float rho, cst;       // xi(line) = maj * rho + cst: the cell's first boundary in minor edge units
+    float G;              // sdd/du * |major direction| * minor pitch
+    float kk;             // slope of that boundary (arc)
+    float dconst, cmaj, dd;  // uniform: d of edge j of a line = maj * cmaj + dconst + j * dd
+    float tconst, tmaj, dt;  // uniform: t likewise (arc)
+    float h, hd;          // SF: the corners sit at xi +- h with denominators +- hd
+    float smin, smaj;     // uniform: minor / major coordinate of the source, negated
+};
+
+// the staged lines m0 .. m0 + nl - 1 (pitch P words, first word pixel jb) walked by every lane
+template <int FOOT, bool ARC, int K>
+__device__ __forceinline__ float fan_lines(const FanLane& L, const float* buf, int P, int jb, int m0, int nl, float wmaj,
+                                           float dmaj, float inv3) {
+    float acc = 0.f;
+    const float ah = FOOT == F2_TF ? fabsf(L.h) : 0.f;
+    const float dden = ARC ? fmaf(L.kk, L.dt, L.dd) : L.dd;
+    const float gh = FOOT == F2_TF ? L.G * L.h : 0.f;
+    // the chunk's first line, and what one line adds to xi and to d (d + k t on an arc)
+    const float maj = (float(m0) + wmaj) * dmaj;
+    const float xi0 = fmaf(maj, L.rho, L.cst), dxi = L.rho * dmaj;
+    float den0 = fmaf(maj, L.cmaj, L.dconst), dl = L.cmaj * dmaj;
+    if constexpr (ARC) {
+        den0 = fmaf(L.kk, fmaf(maj, L.tmaj, L.tconst), den0);
+        dl = fmaf(L.kk, L.tmaj * dmaj, dl);
+    }
+    const float fjb = float(jb), top = float(P - K);
+#pragma unroll 2
+    for (int i = 0; i < nl; ++i) {
+        const float fi = float(i);
+        const float xi = fmaf(fi, dxi, xi0);
+        const float jf = floorf(xi - ah);
+        const float fr = jf - xi;
+        const float* pq = buf + (i * P + (int)__builtin_amdgcn_fmed3f(jf - fjb, 0.f, top));
+        const float den = fmaf(jf, dden, fmaf(fi, dl, den0));
+        float s = pq[K - 1];
+#pragma unroll
+        for (int k = 1; k < K; ++k) {
+            const float dk = fmaf(float(k), dden, den), num = fmaf(fr, L.G, float(k) * L.G);
+            float c;
+            auto edge = [&](float nu_, float de_) {
+                float f = nu_ * frcp(de_);
+                if constexpr (ARC) f = fmaf(f * f, -inv3 * f, f);  // sdd/du atan(f du/sdd)
+                return f;
+            };
+            if constexpr (FOOT == F2_DD) {
+                c = clamp01(edge(num, dk));
+            } else {
+                const float e0 = edge(num - gh, dk + L.hd), e1 = edge(num + gh, dk - L.hd);
+                const float ea = fminf(e0, e1), eb = fmaxf(e0, e1);
+                // 1 - integral over [0, 1] of the ramp from ea to eb
+                const float i2 = 0.5f * frcp(fmaxf(eb - ea, 1.0e-20f));
+                const float z1 = __builtin_amdgcn_fmed3f(1.f, ea, eb) - ea, z0 = __builtin_amdgcn_fmed3f(0.f, ea, eb) - ea;
+                c = 1.f - ((z1 - z0) * (z1 + z0) * i2 + fmaxf(1.f - eb, 0.f) - fmaxf(-eb, 0.f));
+            }
+            s = fmaf(c, pq[k - 1] - pq[k], s);
+        }
+        acc += s;
+    }
+    return acc;
+}
+
+// the walks of one tile over share `share` of `nshares` of the lines
+template <class Tin, int FOOT, bool ARC>
+__device__ __forceinline__ float fan_tile(const Geom<float>& g, const View<float>& v, int ut, const Tin* __restrict__ img,
+                                          int exhaustive, int share, int nshares, float* buf) {
+    const int lane = lane_id();
+    const float pm = fmaxf(g.dx, g.dy);
+    const float inv3 = ARC ? uni(1.f / (g.sdd_du * g.sdd_du * 3.f)) : 0.f;
+    const int iu_a = ut * kW2;
+    const float kA = uni(u_to_slope(g, float(iu_a) - 0.5f)), kB = uni(u_to_slope(g, float(iu_a + kW2) - 0.5f));
+    // direction of the tile's outer rays: X = s + k c, Y = c - k s
+    const float XA = fmaf(kA, v.c, v.s), XB = fmaf(kB, v.c, v.s), YA = fmaf(-kA, v.s, v.c), YB = fmaf(-kB, v.s, v.c);
+    const float fx = FOOT == F2_DD ? 1.f : g.dy, fy = FOOT == F2_DD ? 1.f : g.dx;
+    // a pixel on a ray may lie a pixel beside it
+    const float reach = 0.5f * (float(g.nx) * g.dx + float(g.ny) * g.dy) + fabsf(g.wx + 0.5f * float(g.nx - 1)) * g.dx +
+                        fabsf(g.wy + 0.5f * float(g.ny - 1)) * g.dy;
+    const float m = 1.f + 4.f * pm * frcp(fmaxf(g.sad - reach, 2.f * pm));
+    const bool row = uni((int)(fabsf(XA) * fx <= fabsf(YA) * fy * m || fabsf(XB) * fx <= fabsf(YB) * fy * m)) != 0;
+    const bool col = uni((int)(fabsf(YA) * fy <= fabsf(XA) * fx * m || fabsf(YB) * fy <= fabsf(XB) * fx * m)) != 0;
+    const bool gen = (row && col) || (FOOT == F2_TF && g.dx != g.dy);
+    float acc = 0.f;
+#pragma unroll 1
+    for (int w = row ? 0 : 1; w < (col ? 2 : 1); ++w) {
+        const bool rm = w == 0;
+        const int nmin = rm ? g.nx : g.ny, nmaj = rm ? g.ny : g.nx;
+        const float dmin = rm ? g.dx : g.dy, dmaj = rm ? g.dy : g.dx;
+        const float wmin = rm ? g.wx : g.wy, wmaj = rm ? g.wy : g.wx;
+        FanLane L;
+        const float cmin = rm ? v.s : v.c, tmin = rm ? v.c : -v.s;
+        L.cmaj = rm ? v.c : v.s;
+        L.tmaj = rm ? -v.s : v.c;
+        L.smin = uni(g.sad * cmin);
+        L.smaj = uni(g.sad * L.cmaj);
+        // u grows along the minor axis: the first boundary is the cell's lower edge, else its upper
+        const bool up = uni((int)(rm ? YA > 0.f : XA < 0.f)) != 0;
+        L.kk = u_to_slope(g, float(iu_a + lane) + (up ? -0.5f : 0.5f));
+        {
+            const float X = fmaf(L.kk, v.c, v.s), Y = fmaf(-L.kk, v.s, v.c);
+            const float a = rm ? Y : X, b = rm ? X : Y;
+            const float ia = 1.f / (a * dmin);
+            L.rho = b * ia;
+            L.cst = (rm ? L.kk : -L.kk) * g.sad * ia + (0.5f - wmin);
+            L.G = g.sdd_du * fabsf(a) * dmin;
+        }
+        L.dd = uni(dmin * cmin);
+        L.dconst = uni(fmaf(wmin - 0.5f, L.dd, g.sad));
+        L.dt = uni(dmin * tmin);
+        L.tconst = uni((wmin - 0.5f) * L.dt);
+        L.h = 0.5f * dmaj * L.rho;
+        L.hd = 0.5f * dmaj * (ARC ? fmaf(L.kk, L.tmaj, L.cmaj) : L.cmaj);
+        // the tile's first and last boundaries; the pixels a cell can meet, at the tile's ends and
+        // the first and last line (the width is monotone along the tile and linear along the lines)
+        const float rho0 = rdl(L.rho, 0), rho1 = rdl(L.rho, kW2 - 1), cst0 = rdl(L.cst, 0), cst1 = rdl(L.cst, kW2 - 1);
+        const float y0 = wmaj * dmaj, y1 = (float(nmaj - 1) + wmaj) * dmaj;
+        const float hm = FOOT == F2_TF ? uni(fmaxf(fabsf(rdl(L.h, 0)), fabsf(rdl(L.h, kW2 - 1)))) : 0.f;
+        auto width = [&](int l0, int l1, float y) {
+            return fabsf(fmaf(y, rdl(L.rho, l1) - rdl(L.rho, l0), rdl(L.cst, l1) - rdl(L.cst, l0)));
+        };
+        const float wpx = fmaf(fmaxf(fmaxf(width(0, 1, y0), width(0, 1, y1)),
+                                     fmaxf(width(kW2 - 2, kW2 - 1, y0), width(kW2 - 2, kW2 - 1, y1))),
+                               1.05f, 2.f * hm + 0.01f);
+        const int K = uni(wpx <= 1.f ? 2 : wpx <= 2.f ? 3 : 4);
+        // staged width of one line, its drift from line to line, and the lines per chunk
+        const float span = fmaxf(width(0, kW2 - 1, y0), width(0, kW2 - 1, y1)) + 2.f * hm + float(K + 4);
+        const float drift = fmaxf(fabsf(rho0), fabsf(rho1)) * dmaj;
+        const int lg = uni(span + 16.f * drift <= 100.f ? 4 : 3);  // log2 of the lines per chunk
+        const int NL = 1 << lg, P = lg == 4 ? 100 : 196;           // pitches are 4 mod 64: no bank conflicts
+        const int rounds = uni(min((int)span, P - 1) / kW2 + 1);   // 64-pixel loads per line
+        const int mb = nmaj * share / nshares, me = nmaj * (share + 1) / nshares;
+        for (int m0 = mb; m0 < me; m0 += NL) {
+            const int nl = min(NL, me - m0);
+            // minor range that the chunk's lines can read
+            const float ya = (float(m0) + wmaj) * dmaj, yb = (float(m0 + nl - 1) + wmaj) * dmaj;
+            const float x00 = fmaf(ya, rho0, cst0), x01 = fmaf(ya, rho1, cst1);
+            const float x10 = fmaf(yb, rho0, cst0), x11 = fmaf(yb, rho1, cst1);
+            const float xlo = fminf(fminf(x00, x01), fminf(x10, x11)) - hm;
+            const float xhi = fmaxf(fmaxf(x00, x01), fmaxf(x10, x11)) + hm;
+            if (!exhaustive && (xhi < -float(K) || xlo > float(nmin))) continue;  // beside the image
+            // (clamped so that chunks far outside the image convert to integers)
+            const int jb = uni((int)floorf(__builtin_amdgcn_fmed3f(xlo, -1.0e6f, 1.0e6f)) - 1);
+            // hypot(X, Y) / max(|X|, |Y|) * pixel at minor coordinate mn of the line at major
+            // coordinate mj from the source (rmj = 1 / mj)
+            auto weighed = [&](auto gen_k, float mn, float pix, float mj, float rmj) -> float {
+                if constexpr (decltype(gen_k)::value) {
+                    const float am = fabsf(mn), aj = fabsf(mj);
+                    // (DD: the x edges where |Y| > |X|, as the reference's cos > sin; SF: the
+                    // walk whose edges' corners keep their order)
+                    const float l = FOOT == F2_DD ? aj : aj * dmin, r = FOOT == F2_DD ? am : am * dmaj;
+                    pix = (rm ? l > r : l >= r) ? pix : 0.f;
+                    return pix * (fsqrt(fmaf(mn, mn, mj * mj)) * frcp(fmaxf(am, aj)));
+                } else {
+                    const float q = mn * rmj;
+                    return pix * fsqrt(fmaf(q, q, 1.f));
+                }
+            };
+            // minor and major coordinate of pixel 0 from the source.  Both walks form a pixel's
+            // coordinates with the same operations, so that on the diagonal exactly one keeps it
+            const float cmn = uni(fmaf(wmin, dmin, L.smin)), cmj = uni(fmaf(wmaj, dmaj, L.smaj));
+            // pixels outside the image read zero through the resources' ranges (a line's, or the
+            // image's where a column index runs along the lines of a chunk)
+            auto fill = [&](auto gen_k) {
+                if (rm) {
+                    // lane i: first pixel and major coordinate of line m0 + i; then four lines of
+                    // 64 pixels at a time (lines past the chunk read and store zeros)
+                    const float yl = (float(m0 + lane) + wmaj) * dmaj;
+                    const float xs = fminf(fmaf(yl, rho0, cst0), fmaf(yl, rho1, cst1)) - hm;
+                    const int first = max(jb, (int)floorf(__builtin_amdgcn_fmed3f(xs, -1.0e6f, 1.0e6f)) - 1);
+                    const float mjl = fmaf(float(m0 + lane), dmaj, cmj), rmjl = frcp(mjl);
+                    for (int c = 0; c < rounds; ++c) {
+                        const Tin* line = img + (size_t)m0 * g.nx;
+                        const int lc = c * kW2 + lane;
+                        int row = -jb * 4;  // bytes from pixel 0's word to the line's first word
+                        for (int i0 = 0; i0 < nl; i0 += 4) {
+                            Tin pv[4];
+                            int jj[4];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                jj[e] = rdl_i(first, i0 + e) + lc;
+                                pv[e] = buf_ld<Tin>(buf_rsrc(line, i0 + e < nl ? g.nx * (int)sizeof(Tin) : 0),
+                                                    jj[e] * (int)sizeof(Tin));
+                                line += g.nx;
+                            }
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const float w = weighed(gen_k, fmaf(float(jj[e]), dmin, cmn), to_f(pv[e]), rdl(mjl, i0 + e),
+                                                        rdl(rmjl, i0 + e));
+                                // pixels past the pitch fall on its last word, which no cell reads
+                                *(float*)((char*)buf + (row + min(jj[e] * 4, (jb + P - 1) * 4))) = w;
+                                row += P * 4;
+                            }
+                        }
+                    }
+                } else {
+                    // NL neighbouring image columns of 64 / NL rows per load, four loads at a time
+                    const int i = lane & (NL - 1), dr = kW2 >> lg;
+                    const float mj = fmaf(float(m0 + i), dmaj, cmj), rmj = frcp(mj);
+                    const int jn = uni(min(P, (int)fminf(xhi - xlo, 1.0e6f) + K + 4));
+                    const auto rs = buf_rsrc(img, g.nx * g.ny * (int)sizeof(Tin));
+                    const int step = dr * g.nx * (int)sizeof(Tin);
+                    int r = lane >> lg;
+                    int off = ((jb + r) * g.nx + (m0 + i)) * (int)sizeof(Tin);
+                    float* dst = buf + i * P;
+                    for (int r0 = 0; r0 < jn; r0 += 4 * dr) {
+                        Tin pv[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) pv[e] = buf_ld<Tin>(rs, off + e * step);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            dst[min(r + e * dr, P - 1)] = weighed(gen_k, fmaf(float(jb + r + e * dr), dmin, cmn), to_f(pv[e]), mj, rmj);
+                        r += 4 * dr;
+                        off += 4 * step;
+                    }
+                }
+            };
+            if (gen) fill(std::true_type{});
+            else fill(std::false_type{});
+            __builtin_amdgcn_wave_barrier();
+            if (K == 2) acc += fan_lines<FOOT, ARC, 2>(L, buf, P, jb, m0, nl, wmaj, dmaj, inv3);
+            else if (K == 3) acc += fan_lines<FOOT, ARC, 3>(L, buf, P, jb, m0, nl, wmaj, dmaj, inv3);
+            else acc += fan_lines<FOOT, ARC, 4>(L, buf, P, jb, m0, nl, wmaj, dmaj, inv3);
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    return acc * (g.dx * 0.1f);
+}
+
+// ---------------------------------------------------------------------------------
+// forward, candidate form (FP64, and geometries outside the line walk): candidate
 // pixels of the strip are evaluated 64 at a time (one per lane) into LDS entries, and
 // every tile cell notes the first and the last entry whose footprint covers it (LDS
 // min / max, order-free).  Each lane then walks the entries of its own cell range in
@@ -167,8 +432,20 @@ __device__ __forceinline__ T combine_shares(T (*part)[kW2], int wv, int lane) {
 // S waves share a (view, tile) item, each walking 1/S of the strip's lines; the partial
 // sums are added in a fixed order.  S = 4 when the items alone would leave the chip
 // with few waves.
-template <class Tin, class Tout, class T, int FOOT, int S>
-__global__ __launch_bounds__(256) void fbct_proj_kernel(Geom<T> g, const View<T>* __restrict__ views, int vstride,
+// FORM 0: candidates; 1: line walk, flat detector; 2: line walk, arc
+template <class Tin, class T, int FOOT, int FORM>
+__device__ __forceinline__ T fbct_proj_item(const Geom<T>& g, const View<T>& v, int ut, const Tin* __restrict__ img,
+                                            int exhaustive, int share, int nshares) {
+    if constexpr (FORM == 0) {
+        return fbct_proj_acc<Tin, T, FOOT>(g, v, ut, img, exhaustive, share, nshares);
+    } else {
+        __shared__ __align__(16) float buf[4][kFanWords];
+        return fan_tile<Tin, FOOT, FORM == 2>(g, v, ut, img, exhaustive, share, nshares, buf[threadIdx.x / kW2]);
+    }
+}
+
+template <class Tin, class Tout, class T, int FOOT, int S, int FORM>
+__global__ __launch_bounds__(256, FORM ? kFanWaves : 1) void fbct_proj_kernel(Geom<T> g, const View<T>* __restrict__ views, int vstride,
                                                         int nviews, const Tin* __restrict__ img,
                                                         Tout* __restrict__ proj, int exhaustive) {
     __shared__ T part[4][kW2];
@@ -184,7 +461,7 @@ __global__ __launch_bounds__(256) void fbct_proj_kernel(Geom<T> g, const View<T>
         // the view in registers (a wave-uniform index: scalar loads, once per item), so that
         // the walk's LDS atomics and barriers do not make the compiler reload it every batch
         const View<T> vw = views[(size_t)uni(b) * vstride];
-        acc = fbct_proj_acc<Tin, T, FOOT>(g, vw, ut, img, exhaustive, wv % S, S);
+        acc = fbct_proj_item<Tin, T, FOOT, FORM>(g, vw, uni(ut), img, exhaustive, wv % S, S);
     }
     if (S > 1) {
         part[wv][lane] = acc;
@@ -296,8 +573,8 @@ __device__ __forceinline__ int find_slice(const Slice2<T>* __restrict__ sl, int 
 // of a block (S = 1, 2, 4; the shares are added in a fixed order); the back pass splits
 // each (slice, row, 64-pixel) item's views over VS waves (VS = 1, 2, 4).  A block is
 // always 4 waves and holds 4/S (4/VS) items.
-template <class Tin, class Tout, class T, int FOOT, int S>
-__global__ __launch_bounds__(256) void fbct_proj_batch_kernel(const Slice2<T>* __restrict__ sl, int nslices,
+template <class Tin, class Tout, class T, int FOOT, int S, int FORM>
+__global__ __launch_bounds__(256, FORM ? kFanWaves : 1) void fbct_proj_batch_kernel(const Slice2<T>* __restrict__ sl, int nslices,
                                                               int nitems, const Tin* __restrict__ img,
                                                               Tout* __restrict__ proj) {
     __shared__ T part[4][kW2];
@@ -323,7 +600,7 @@ __global__ __launch_bounds__(256) void fbct_proj_batch_kernel(const Slice2<T>* _
         ut = uni(tile_by_rank(local / s.nviews, min(max((int)floor(-g.wu / T(kW2)), 0), nut - 1), nut));
         b = uni(local % s.nviews);
         const View<T> vw = s.views[b];
-        acc = fbct_proj_acc<Tin, T, FOOT>(g, vw, ut, img + s.img_off, 0, wv % S, S);
+        acc = fbct_proj_item<Tin, T, FOOT, FORM>(g, vw, ut, img + s.img_off, 0, wv % S, S);
     }
     if (S > 1) {
         part[wv][lane] = acc;
@@ -385,29 +662,68 @@ __global__ __launch_bounds__(256) void fbct_back_batch_kernel(const Slice2<T>* _
 // ===================================================================================
 namespace ctsim {
 
+// Whether the line walk covers every tile of a geometry: the source beyond the image for
+// every ray's walk, cells of at most three pixels along a line (soft edges included) and a
+// tile's line within the staged pitch.  phi bounds the angle between a ray and the walk's
+// major axis: the split at |X| = |Y| (SF: |X| dy = |Y| dx), the tile that straddles it and
+// the pixel beside the ray.
+bool fan_walk_ok(const Geom<float>& g, int kind) {
+    if (!(g.dx > 0.f && g.dy > 0.f && g.du > 0.f && g.sdd > 0.f && g.sdd_du > 50.f)) return false;
+    if ((double)g.nx * g.ny > 1.0e8) return false;  // image offsets in 32 bits, chunks outside it included
+    const double dx = g.dx, dy = g.dy, pm = std::max(dx, dy), da = (double)g.du / g.sdd;
+    const double ex = 0.5 * g.nx * dx + std::fabs(g.wx + 0.5 * (g.nx - 1)) * dx + pm;
+    const double ey = 0.5 * g.ny * dy + std::fabs(g.wy + 0.5 * (g.ny - 1)) * dy + pm;
+    const double R = ex + ey, sad = g.sad;
+    if (!(sad > R + 4.0 * pm)) return false;
+    const int cells = (g.nu + kW2 - 1) / kW2 * kW2;
+    const double um = std::max(std::fabs(g.wu - 0.5), std::fabs(g.wu + cells + 0.5)) * da;
+    const double gam = g.dettype == 1 ? std::atan(um) : um;
+    const double slack = kW2 * da + 4.0 * pm / (sad - R);
+    for (int w = 0; w < 2; ++w) {
+        const double dmin = w == 0 ? dx : dy, dmaj = w == 0 ? dy : dx;
+        const double phi = (kind == F2_DD ? 0.78539816339744831 : std::atan2(dmin, dmaj)) + slack;
+        if (!(phi + gam < 1.4)) return false;
+        if (!(sad * std::cos(phi + gam) > (w == 0 ? ey : ex) + 4.0 * pm)) return false;
+        const double wpx = (sad + R) / std::cos(phi) * da / dmin, h = kind == F2_DD ? 0.0 : std::tan(phi) * dmaj / dmin;
+        if (!(1.05 * wpx + h + 0.01 <= 3.0)) return false;
+        if (!(kW2 * wpx + h + 8.0 + 8.0 * std::tan(phi) * dmaj / dmin <= 196.0)) return false;
+    }
+    return true;
+}
+
+template <class Tin, class Tout, class T, int FOOT, int S>
+static void proj2_form(unsigned blocks, hipStream_t st, const Geom<T>& g, const View<T>* views, int vstride, int nviews,
+                       const void* img, void* proj, int exhaustive) {
+#define CT_P2(F)                                                                                                        \
+    hipLaunchKernelGGL((fbct_proj_kernel<Tin, Tout, T, FOOT, S, F>), dim3(blocks), dim3(256), 0, st, g, views, vstride, \
+                       nviews, (const Tin*)img, (Tout*)proj, exhaustive)
+    if constexpr (sizeof(T) == 4) {
+        if (fan_walk_ok(g, FOOT)) {
+            if (g.dettype == 1) CT_P2(1);
+            else CT_P2(2);
+            return;
+        }
+    }
+    CT_P2(0);
+#undef CT_P2
+}
+
 template <class Tin, class Tout, class T>
 static hipError_t proj2(const Geom<T>& g, const View<T>* views, int vstride, int nviews, const void* img, void* proj,
                         int kind, int exhaustive, hipStream_t st) {
     const long long nut = (g.nu + kW2 - 1) / kW2;
     const long long items = (long long)nviews * nut;
     if (items == 0) return hipSuccess;
-    if (items < kFewItems2D) {
-        const unsigned blocks = (unsigned)items;
-        if (kind == F2_DD)
-            hipLaunchKernelGGL((fbct_proj_kernel<Tin, Tout, T, F2_DD, 4>), dim3(blocks), dim3(256), 0, st, g, views,
-                               vstride, nviews, (const Tin*)img, (Tout*)proj, exhaustive);
-        else
-            hipLaunchKernelGGL((fbct_proj_kernel<Tin, Tout, T, F2_TF, 4>), dim3(blocks), dim3(256), 0, st, g, views,
-                               vstride, nviews, (const Tin*)img, (Tout*)proj, exhaustive);
-        return hipGetLastError();
-    }
-    const unsigned blocks = (unsigned)((items + 3) / 4);
-    if (kind == F2_DD)
-        hipLaunchKernelGGL((fbct_proj_kernel<Tin, Tout, T, F2_DD, 1>), dim3(blocks), dim3(256), 0, st, g, views, vstride,
-                           nviews, (const Tin*)img, (Tout*)proj, exhaustive);
-    else
-        hipLaunchKernelGGL((fbct_proj_kernel<Tin, Tout, T, F2_TF, 1>), dim3(blocks), dim3(256), 0, st, g, views, vstride,
-                           nviews, (const Tin*)img, (Tout*)proj, exhaustive);
+    const bool few = items < kFewItems2D;
+    const unsigned blocks = few ? (unsigned)items : (unsigned)((items + 3) / 4);
+#define CT_P2S(F)                                                                                             \
+    do {                                                                                                      \
+        if (few) proj2_form<Tin, Tout, T, F, 4>(blocks, st, g, views, vstride, nviews, img, proj, exhaustive); \
+        else proj2_form<Tin, Tout, T, F, 1>(blocks, st, g, views, vstride, nviews, img, proj, exhaustive);    \
+    } while (0)
+    if (kind == F2_DD) CT_P2S(F2_DD);
+    else CT_P2S(F2_TF);
+#undef CT_P2S
     return hipGetLastError();
 }
 
@@ -483,18 +799,25 @@ hipError_t fbct_back_launch<double>(const Geom<double>& g, const View<double>* v
 size_t slice2_size(bool dbl) { return dbl ? sizeof(Slice2<double>) : sizeof(Slice2<float>); }
 
 template <class Tin, class Tout, class T, int FOOT, int S>
-static void proj2b_s(const void* sl, int nslices, int nitems, const void* img, void* proj, hipStream_t st) {
+static void proj2b_s(const void* sl, int nslices, int nitems, const void* img, void* proj, int form, hipStream_t st) {
     const unsigned blocks = (unsigned)(((long long)nitems * S + 3) / 4);
-    hipLaunchKernelGGL((fbct_proj_batch_kernel<Tin, Tout, T, FOOT, S>), dim3(blocks), dim3(256), 0, st,
-                       (const Slice2<T>*)sl, nslices, nitems, (const Tin*)img, (Tout*)proj);
+#define CT_P2B(F)                                                                                        \
+    hipLaunchKernelGGL((fbct_proj_batch_kernel<Tin, Tout, T, FOOT, S, F>), dim3(blocks), dim3(256), 0, st, \
+                       (const Slice2<T>*)sl, nslices, nitems, (const Tin*)img, (Tout*)proj)
+    if constexpr (sizeof(T) == 4) {
+        if (form == 1) { CT_P2B(1); return; }
+        if (form == 2) { CT_P2B(2); return; }
+    }
+    CT_P2B(0);
+#undef CT_P2B
 }
 
 template <class Tin, class Tout, class T>
 static hipError_t proj2b(const void* sl, int nslices, int nitems, const void* img, void* proj, int kind, int split,
-                         hipStream_t st) {
+                         int form, hipStream_t st) {
     if (nitems == 0) return hipSuccess;
     if (split != 1 && split != 2 && split != 4) return hipErrorInvalidValue;
-#define CT_P2B(F, S) proj2b_s<Tin, Tout, T, F, S>(sl, nslices, nitems, img, proj, st)
+#define CT_P2B(F, S) proj2b_s<Tin, Tout, T, F, S>(sl, nslices, nitems, img, proj, form, st)
     if (kind == F2_DD) {
         if (split == 1) CT_P2B(F2_DD, 1); else if (split == 2) CT_P2B(F2_DD, 2); else CT_P2B(F2_DD, 4);
     } else {
@@ -531,10 +854,10 @@ static hipError_t back2b(const void* sl, int nslices, int nitems, const void* pr
 
 template <>
 hipError_t fbct_proj_batch_launch<float>(const void* sl, int nslices, int nitems, const void* img, int img_dt,
-                                         void* proj, int proj_dt, int kind, int split, hipStream_t st) {
-#define OUT_F32(TI) return proj2b<TI, float, float>(sl, nslices, nitems, img, proj, kind, split, st)
-#define OUT_F16(TI) return proj2b<TI, __half, float>(sl, nslices, nitems, img, proj, kind, split, st)
-#define OUT_BF16(TI) return proj2b<TI, __hip_bfloat16, float>(sl, nslices, nitems, img, proj, kind, split, st)
+                                         void* proj, int proj_dt, int kind, int split, int form, hipStream_t st) {
+#define OUT_F32(TI) return proj2b<TI, float, float>(sl, nslices, nitems, img, proj, kind, split, form, st)
+#define OUT_F16(TI) return proj2b<TI, __half, float>(sl, nslices, nitems, img, proj, kind, split, form, st)
+#define OUT_BF16(TI) return proj2b<TI, __hip_bfloat16, float>(sl, nslices, nitems, img, proj, kind, split, form, st)
     switch (proj_dt) {
         case DT_F32: CT_DISPATCH_IN(img_dt, OUT_F32);
         case DT_F16: CT_DISPATCH_IN(img_dt, OUT_F16);
@@ -548,9 +871,9 @@ hipError_t fbct_proj_batch_launch<float>(const void* sl, int nslices, int nitems
 
 template <>
 hipError_t fbct_proj_batch_launch<double>(const void* sl, int nslices, int nitems, const void* img, int img_dt,
-                                          void* proj, int proj_dt, int kind, int split, hipStream_t st) {
+                                          void* proj, int proj_dt, int kind, int split, int form, hipStream_t st) {
     if (img_dt != DT_F64 || proj_dt != DT_F64) return hipErrorInvalidValue;
-    return proj2b<double, double, double>(sl, nslices, nitems, img, proj, kind, split, st);
+    return proj2b<double, double, double>(sl, nslices, nitems, img, proj, kind, split, form, st);
 }
 
 template <>

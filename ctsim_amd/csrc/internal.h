@@ -94,7 +94,10 @@ struct Slice2 {
 
 template <class T>
 hipError_t fbct_proj_batch_launch(const void* slices, int nslices, int nitems, const void* img, int img_dt,
-                                  void* proj, int proj_dt, int kind, int split, hipStream_t st);
+                                  void* proj, int proj_dt, int kind, int split, int form, hipStream_t st);
+// whether the FP32 forward's line walk covers a geometry (kind as above); a batch takes one
+// form for all of its slices: 0 candidates, 1 line walk (flat), 2 line walk (arc)
+bool fan_walk_ok(const Geom<float>& g, int kind);
 template <class T>
 hipError_t fbct_back_batch_launch(const void* slices, int nslices, int nitems, const void* proj, int proj_dt,
                                   void* img, int img_dt, int kind, int split, hipStream_t st);
