@@ -478,12 +478,129 @@ __global__ __launch_bounds__(256, FORM ? kFanWaves : 1) void fbct_proj_kernel(Ge
 // consecutive pixels of a row; the 4 waves of a block split the views into four
 // contiguous ranges and their partial sums are added in a fixed order.
 // ---------------------------------------------------------------------------------
+// One view's matched backprojection of pixel (xc, yc), FP32: amp * sum_i w_i row_i.  The
+// first three footprint cells are loaded at once through the row's resource (cells past the
+// detector read zero), wider footprints loop over the rest.
+//   amp = dx hypot(X, Y) / max(|X|, |Y|) / 10, (X, Y) the pixel relative to the source: the
+//     ray's cosines are |Y| and |X| over hypot(X, Y), so no normalised direction is formed;
+//   DD: cell k of [lo, hi] weighs min(hi, k + 1) - max(lo, k);
+//   SF: cell k weighs C(k + 1) - C(k), C the trapezoid's running integral, the difference of
+//     its two ramps' integrals; two reciprocals per pixel where the per-cell form takes two
+//     per cell.
+// Bound by instruction issue: 96 -> 55 (DD) vector instructions per 64 pixel-views, with the
+// views through scalar loads.  256^2, 360 views, DD: 75 -> 43 us; 64 uneven FP16 slices:
+// 7.97 -> 4.37 ms.
+// The cells are returned as loaded: the caller evaluates a second view's footprint before it
+// uses them.
+template <class Tin>
+struct BackView {
+    Tin p0, p1, p2;
+    float w0, w1, w2, rest;  // weights times amp; the sum of the cells past the third
+};
+template <class Tin, int KIND>
+__device__ __forceinline__ BackView<Tin> fbct_back_view(const Geom<float>& g, const View<float>& v, float xc, float yc,
+                                                        const Tin* __restrict__ row) {
+    const float t = xc * v.c - yc * v.s, d = fmaf(yc, v.c, fmaf(xc, v.s, g.sad));
+    const float X = fabsf(fmaf(g.sad, v.s, xc)), Y = fabsf(fmaf(g.sad, v.c, yc));
+    const float amp = fsqrt(fmaf(X, X, Y * Y)) * frcp(fmaxf(X, Y)) * (g.dx * 0.1f);
+    const float fn = float(g.nu);
+    const float half = 0.5f - g.wu;
+    auto det = [&](float num, float den) {
+        const float q = num * frcp(den);
+        return fmaf(g.sdd_du, g.dettype == 1 ? q : atanf(q), half);
+    };
+    float lo, hi, t0 = 0.f, t1 = 0.f, t2 = 0.f, t3 = 0.f;
+    if constexpr (KIND == 0) {
+        const bool xdom = Y > X;
+        // (through uni, so that the choice is made between registers and not between addresses)
+        const float a = xdom ? uni(v.dxc2) : uni(v.dys2), b = xdom ? uni(v.dxs2) : uni(v.ndyc2);
+        const float u0 = det(t + a, d + b), u1 = det(t - a, d - b);
+        lo = fminf(u0, u1);
+        hi = fmaxf(u0, u1);
+    } else {
+        const float ax = v.dxc2 + v.dys2, bx = v.dxs2 + v.ndyc2, ay = v.dxc2 - v.dys2, by = v.dxs2 - v.ndyc2;
+        t0 = det(t + ax, d + bx);
+        t1 = det(t - ay, d - by);
+        t2 = det(t + ay, d + by);
+        t3 = det(t - ax, d - bx);
+        cswap(t0, t1);
+        cswap(t2, t3);
+        cswap(t0, t2);
+        cswap(t1, t3);
+        cswap(t1, t2);
+        lo = t0;
+        hi = t3;
+    }
+    const float cl = __builtin_amdgcn_fmed3f(lo, 0.f, fn), ch = __builtin_amdgcn_fmed3f(hi, 0.f, fn);
+    const int ilo = (int)cl;  // cl >= 0: truncation is floor
+    const float f = __builtin_amdgcn_fractf(cl), fi = cl - f, h = ch - fi;
+    const auto rs = buf_rsrc(row, g.nu * (int)sizeof(Tin));
+    const int off = ilo * (int)sizeof(Tin);
+    BackView<Tin> r;
+    r.p0 = buf_ld<Tin>(rs, off);
+    r.p1 = buf_ld<Tin>(rs, off + (int)sizeof(Tin));
+    r.p2 = buf_ld<Tin>(rs, off + 2 * (int)sizeof(Tin));
+    float s = 0.f;
+    if constexpr (KIND == 0) {
+        r.w0 = (fminf(h, 1.f) - f) * amp;
+        r.w1 = clamp01(h - 1.f) * amp;
+        r.w2 = clamp01(h - 2.f) * amp;
+        if (h > 3.f)
+            for (int k = 3; float(k) < h; ++k) s += fminf(h - float(k), 1.f) * to_f(buf_ld<Tin>(rs, off + k * (int)sizeof(Tin)));
+    } else {
+        const float ia = 0.5f * frcp(fmaxf(t1 - t0, 1.0e-20f)), ib = 0.5f * frcp(fmaxf(t3 - t2, 1.0e-20f));
+        // integral of the trapezoid up to cell edge fi + k
+        auto cum = [&](float k) {
+            const float e = fi + k;
+            const float a = __builtin_amdgcn_fmed3f(e, t0, t1) - t0, b = __builtin_amdgcn_fmed3f(e, t2, t3) - t2;
+            return fmaf(a * a, ia, fmaxf(e - t1, 0.f)) - fmaf(b * b, ib, fmaxf(e - t3, 0.f));
+        };
+        float c0 = cum(0.f);  // zero unless the footprint starts before the detector
+        const float c1 = cum(1.f), c2 = cum(2.f);
+        float c3 = cum(3.f);
+        r.w0 = (c1 - c0) * amp;
+        r.w1 = (c2 - c1) * amp;
+        r.w2 = (c3 - c2) * amp;
+        if (h > 3.f)
+            for (int k = 3; float(k) < h; ++k) {
+                c0 = c3;
+                c3 = cum(float(k + 1));
+                s += (c3 - c0) * to_f(buf_ld<Tin>(rs, off + k * (int)sizeof(Tin)));
+            }
+    }
+    r.rest = amp * s;
+    return r;
+}
+
+// a view of the table at a wave-uniform index through scalar loads (the pointer of a batch's
+// slice comes from memory, which alone would make them flat vector loads with their latency in
+// every view)
+__device__ __forceinline__ View<float> load_view(const View<float>* p) {
+    const auto* q = (const __attribute__((address_space(4))) float*)(const void*)p;
+    return View<float>{q[0], q[1], q[2], q[3], q[4], q[5], q[6], q[7]};
+}
+
 template <class Tin, class T, int KIND>  // KIND 0 dd, 1 tf, 2 pd
 __device__ __forceinline__ T fbct_back_pixel(const Geom<T>& g, const View<T>* __restrict__ views, int vstride, int b0,
                                              int b1, int ix, int iy, const Tin* __restrict__ proj) {
     T img = T(0);
     if (ix >= g.nx) return img;
     const T xc = (T(ix) + g.wx) * g.dx, yc = (T(iy) + g.wy) * g.dy;
+    if constexpr (KIND != 2 && sizeof(T) == 4) {
+        auto add = [&](const BackView<Tin>& r) {
+            img += fmaf(r.w2, to_f(r.p2), fmaf(r.w1, to_f(r.p1), fmaf(r.w0, to_f(r.p0), r.rest)));
+        };
+        int b = b0;
+        for (; b + 1 < b1; b += 2) {
+            const View<float> v0 = load_view(views + (size_t)b * vstride), v1 = load_view(views + (size_t)(b + 1) * vstride);
+            const BackView<Tin> r0 = fbct_back_view<Tin, KIND>(g, v0, xc, yc, proj + (size_t)b * g.nu);
+            const BackView<Tin> r1 = fbct_back_view<Tin, KIND>(g, v1, xc, yc, proj + (size_t)(b + 1) * g.nu);
+            add(r0);
+            add(r1);
+        }
+        if (b < b1) add(fbct_back_view<Tin, KIND>(g, load_view(views + (size_t)b * vstride), xc, yc, proj + (size_t)b * g.nu));
+        return img;
+    }
     for (int b = b0; b < b1; ++b) {
         const View<T> v = views[(size_t)b * vstride];
         const Tin* row = proj + (size_t)b * g.nu;
@@ -541,7 +658,7 @@ __global__ __launch_bounds__(256) void fbct_back_kernel(Geom<T> g, const View<T>
     const int nxb = (g.nx + kW2 - 1) / kW2;
     const int iy = blockIdx.x / nxb;
     const int ix = (blockIdx.x % nxb) * kW2 + lane_id();
-    const int w = threadIdx.x / kW2;
+    const int w = uni((int)(threadIdx.x / kW2));  // wave-uniform, so that the views come through scalar loads
     const int per = (nviews + 3) / 4;
     const int b0 = min(w * per, nviews), b1 = min(b0 + per, nviews);
     const T s = fbct_back_pixel<Tin, T, KIND>(g, views, vstride, b0, b1, ix, iy, proj);
@@ -634,12 +751,12 @@ __global__ __launch_bounds__(256) void fbct_back_batch_kernel(const Slice2<T>* _
         const Slice2<T>& s = sl[si];
         const Geom<T> g = s.g;
         const View<T>* views = s.views;
-        const int nviews = s.nviews;
+        const int nviews = uni(s.nviews);
         const int local = item - s.item0;
         const int nxb = (g.nx + kW2 - 1) / kW2;
         iy = local / nxb;
         ix = (local % nxb) * kW2 + lane;
-        const int share = wv % VS;
+        const int share = uni(wv % VS);
         const int per = (nviews + VS - 1) / VS;
         const int b0 = min(share * per, nviews), b1 = min(b0 + per, nviews);
         v = fbct_back_pixel<Tin, T, KIND>(g, views, 1, b0, b1, ix, iy, proj + s.sino_off);
