@@ -917,6 +917,440 @@ __global__ __launch_bounds__(WPB * kWave, kRingWaves) void cbct_proj_ring_kernel
 }
 
 // ---------------------------------------------------------------------------------
+// Forward projection, matrix form (FP32 volumes whose voxels are 1/4 to 14 rows thick on the
+// detector everywhere).  The same work items, strips, footprints and row gathers as the ring
+// form; what differs is what happens to a surviving column's 64 RPL row sums.  A tile is
+//     p[cell, row] = sum over columns of w[cell, column] q[column, row],
+// a product whose inner dimension is the strip's columns, so four columns at a time go to the
+// FP32 matrix instruction (16 cells x 4 columns x 16 rows per step) and the tile stays in
+// registers: no LDS accumulators, and one chain per four columns instead of one per column.
+// Lane l works for column l / 16 of its group: it holds that column's parameters in vector
+// registers (the ring form reads ten of them per column with readlane), the weight of cell
+// l % 16, and, in step t, row 16 t + l % 16.
+//
+//  * survivors of a 64-candidate batch are appended to a queue of records in LDS; groups of
+//    four leave it in order and at most three records wait for the next batch, so the sums do
+//    not depend on how candidates fall into batches;
+//  * a group's voxels come with two 16-byte loads per lane and 128 voxels (the ring form: two
+//    4-byte loads per column), issued one group ahead, are scaled by sqrt(r^2 + zc^2) in
+//    registers and staged in LDS with a zero word before and five after each column;
+//  * a zero weight times a value that is not finite would spread it over the tile, so a wave
+//    whose tile ends up with one walks its item again and adds each footprint's own cells only;
+//  * a footprint of more than four tile cells takes a record for every four of them.
+//
+// 45 vector and 6 scalar instructions per column and item against the ring form's 57 and 48
+// (SF, 41 views of 1024 x 64 over 512^2 x 128: 1.47 -> 0.90 ms; 720 views of 1024 x 384 over
+// 512^2 x 256, two row chunks per item: 112 -> 58 ms).  It now waits on memory as much as on
+// issue: each view reads the volume once from beyond L2.
+// ---------------------------------------------------------------------------------
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kRecWords = 12;           // one column's record
+constexpr int kQueue = kWave + 4;       // records a wave can hold: a batch and what it left over
+constexpr int kMatLead = 4, kMatPad = 8;  // words before and after a column's staged voxels
+constexpr int kMatWaves = 4;            // waves per SIMD the kernel is compiled for (five spill: 0.97 against 0.90 ms
+                                        // for a 41-view subset of the 512^2 x 128 volume)
+__host__ __device__ constexpr int mat_wave_words(int nv) { return kQueue * kRecWords + 4 * (kMatLead + nv + kMatPad); }
+
+// sum over the K voxels from ja on of (overlap with the row) * staged value, ja and x_k =
+// x_0 + k zinc as in ring_gather.  With d_k = 1 - c_k = clamp01(1 - x_0 - k zinc) the sum
+// sum_k (d_k - d_{k+1}) v_k is v_0 + sum_{0 < k < K} d_k (v_k - v_{k-1}): d_0 = 1 (or v_0 is the
+// zero word) and d_K = 0.  Voxels past the row add exactly zero, so the sum does not depend on
+// K once (K - 1) zinc >= 1, and a batch may take the largest K of its columns.
+template <int K>
+__device__ __forceinline__ float mat_gather(const float* zs, float jhi, float tt, float rz, float zinc) {
+    const float jf = __builtin_amdgcn_fmed3f(ceilf(fmaf(tt, rz, -1.f)), -1.f, jhi);
+    const float* pz = zs + (int)jf;
+    const float y0 = 1.f - fmaf(jf, zinc, -tt);
+    float s = pz[0];
+#pragma unroll
+    for (int k = 1; k < K; ++k) s = fmaf(clamp01(fmaf(-float(k), zinc, y0)), pz[k] - pz[k - 1], s);
+    return s;
+}
+
+// A column's u footprint and per-column factors, FP32.  With (X, Y) the column relative to the
+// source, the ray's cosines are |Y| and |X| over its length r, so amp / r = dx / max(|cos|,
+// |sin|) / 10 / r = 0.1 dx / max(|X|, |Y|): no direction is normalised and no root taken.
+template <int FOOT>
+struct ColFoot {
+    float p0, p1, p2, p3;  // corners as in col_corners
+    int ilo, ihi;
+    float ampr, r2, d;     // amp / r, r^2, distance along the central ray
+};
+template <int FOOT>
+__device__ __forceinline__ bool col_foot(const Geom<float>& g, const View<float>& v, float xc, float yc, ColFoot<FOOT>& f) {
+    const float t = xc * v.c - yc * v.s, d = g.sad + xc * v.s + yc * v.c;
+    const float X = fabsf(fmaf(g.sad, v.s, xc)), Y = fabsf(fmaf(g.sad, v.c, yc));
+    f.ampr = g.dx * 0.1f * frcp(fmaxf(X, Y));
+    f.r2 = fmaf(t, t, d * d);
+    f.d = d;
+    float lo, hi, clo, chi;
+    if constexpr (FOOT == FOOT_DD) {
+        Column<float> k;
+        k.t = t;
+        k.d = d;
+        k.xdom = Y > X;
+        dd_bounds(k, v, g, lo, hi);
+    } else {
+        Column<float> k;
+        k.t = t;
+        k.d = d;
+        float tau[4];
+        sf_taus(k, v, g, tau);
+        f.p0 = tau[0];
+        f.p1 = tau[1];
+        f.p2 = tau[2];
+        f.p3 = tau[3];
+        lo = tau[0];
+        hi = tau[3];
+    }
+    const bool ok = clamp_cells(lo, hi, g.nu, 16, clo, chi, f.ilo, f.ihi);
+    if constexpr (FOOT == FOOT_DD) {
+        f.p0 = clo;
+        f.p1 = chi;
+    }
+    return ok;
+}
+// weights of the four cells from c0 on, times amp / r.  SF: differences of the trapezoid's
+// running integral at the five cell edges, the integral being that of its rising ramp less that
+// of its falling one: two reciprocals for the four cells where sf_weight takes two per cell
+template <int FOOT>
+__device__ __forceinline__ float4 foot_weights(const ColFoot<FOOT>& f, int c0) {
+    float4 w;
+    if constexpr (FOOT == FOOT_DD) {
+        w.x = u_weight<float, FOOT>(c0 + 0, f.ilo, f.ihi, f.p0, f.p1, 0.f, 0.f) * f.ampr;
+        w.y = u_weight<float, FOOT>(c0 + 1, f.ilo, f.ihi, f.p0, f.p1, 0.f, 0.f) * f.ampr;
+        w.z = u_weight<float, FOOT>(c0 + 2, f.ilo, f.ihi, f.p0, f.p1, 0.f, 0.f) * f.ampr;
+        w.w = u_weight<float, FOOT>(c0 + 3, f.ilo, f.ihi, f.p0, f.p1, 0.f, 0.f) * f.ampr;
+    } else {
+        const float ia = 0.5f * frcp(fmaxf(f.p1 - f.p0, 1.0e-20f)), ib = 0.5f * frcp(fmaxf(f.p3 - f.p2, 1.0e-20f));
+        const float e0 = float(c0) - 0.5f;
+        auto cum = [&](float k) {
+            const float e = e0 + k;
+            const float a = __builtin_amdgcn_fmed3f(e, f.p0, f.p1) - f.p0, b = __builtin_amdgcn_fmed3f(e, f.p2, f.p3) - f.p2;
+            return fmaf(a * a, ia, fmaxf(e - f.p1, 0.f)) - fmaf(b * b, ib, fmaxf(e - f.p3, 0.f));
+        };
+        const float s0 = cum(0.f), s1 = cum(1.f), s2 = cum(2.f), s3 = cum(3.f), s4 = cum(4.f);
+        const int n = f.ihi - c0;  // cells past the footprint's last (a capped one) get nothing
+        w.x = (s1 - s0) * f.ampr;
+        w.y = n >= 1 ? (s2 - s1) * f.ampr : 0.f;
+        w.z = n >= 2 ? (s3 - s2) * f.ampr : 0.f;
+        w.w = n >= 3 ? (s4 - s3) * f.ampr : 0.f;
+    }
+    return w;
+}
+
+// the same sum voxel by voxel, without those that do not overlap the row (values that are not
+// finite stay in the rows of their voxel)
+__device__ __forceinline__ float mat_gather_each(const float* zs, float jhi, float tt, float rz, float zinc) {
+    const float jf = __builtin_amdgcn_fmed3f(ceilf(fmaf(tt, rz, -1.f)), -1.f, jhi);
+    const float* pz = zs + (int)jf;
+    const float y0 = 1.f - fmaf(jf, zinc, -tt);
+    float s = 0.f, d = clamp01(y0);
+#pragma unroll 1
+    for (int k = 0; k < 5; ++k) {
+        const float e = clamp01(fmaf(-float(k + 1), zinc, y0)), w = d - e;
+        if (w > 0.f) s = fmaf(w, pz[k], s);
+        d = e;
+    }
+    return s;
+}
+
+// NV: staged voxels per column (64 or 128, at least the most that an item's rows can need)
+template <class Tout, int FOOT, int SPLIT, int RPL, int NV, int WPB>
+__global__ __launch_bounds__(WPB * kWave, kMatWaves) void cbct_proj_mat_kernel(Geom<float> g, const View<float>* __restrict__ views,
+                                                                       int vstride, int nviews,
+                                                                       const float* __restrict__ vol, unsigned vol_bytes,
+                                                                       const uint8_t* __restrict__ map,
+                                                                       Tout* __restrict__ proj, int exhaustive) {
+    using T = float;
+    constexpr int TU = 16, RT = 4 * RPL, NL = NV / 64;
+    constexpr int kCellW = kWave * RPL;
+    constexpr int kPitch = kMatLead + NV + kMatPad, kWaveW = mat_wave_words(NV);
+    static_assert(SPLIT == 1 || (SPLIT == WPB && WPB * TU * kCellW <= WPB * kWaveW), "the shares' tiles fit the queues' LDS");
+    __shared__ __align__(16) T lds[WPB * kWaveW];
+    const int nut = (g.nu + TU - 1) / TU;
+    const int nvc = (g.nv + kCellW - 1) / kCellW;
+    const int items = nviews * nut * nvc;
+    const int bid = blockIdx.x;
+    const int wv = uni((int)(threadIdx.x / kWave));
+    const int item = SPLIT == 1 ? bid * WPB + wv : bid;
+    const int share = SPLIT == 1 ? 0 : wv;
+    if (item >= items) return;  // SPLIT > 1: the whole block leaves together
+    const int vc = item % nvc;
+    const int b = (item / nvc) % nviews;
+    // longest work first (tiles in order of their distance from the central ray's tile)
+    const int ut = tile_by_rank(item / (nvc * nviews), min(max((int)floor(-g.wu / T(TU)), 0), nut - 1), nut);
+    const int lane = lane_id(), l16 = lane & 15, l4 = lane >> 4;
+    const int iv_a = uni(vc * kCellW), iu_a = uni(ut * TU);
+    const int iu_b = min(iu_a + TU, g.nu) - 1;
+    const View<T> v = views[(size_t)b * vstride];
+    const bool row_major = fabs_t(v.c) >= fabs_t(v.s);
+    const int m_end = row_major ? g.ny : g.nx;
+    const T kL = u_to_slope(g, T(iu_a) - T(0.5));
+    const T kR = u_to_slope(g, T(iu_b) + T(0.5));
+    const int iv_last = min(iv_a + kCellW, g.nv) - 1;
+    T* const queue = lds + wv * kWaveW;
+    T* const stage = queue + kQueue * kRecWords + l4 * kPitch + kMatLead;  // voxel 0 of this lane's column
+    if (l16 < kMatLead) stage[l16 - kMatLead] = T(0);
+    const T wzdz = v.wz * g.dz;
+    const T frow = T(iv_a + l16) - T(0.5);  // lower edge of this lane's row in step 0
+    const T zl = T(4 * l16) * g.dz;         // zc of the lane's first loaded voxel from the column's first
+    const auto rs = buf_rsrc(vol, (int)vol_bytes);
+
+    const T dz64 = uni(T(64) * g.dz);
+
+    f32x4 acc[RT];
+    auto walk = [&](auto careful_k) {
+        constexpr bool careful = decltype(careful_k)::value;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        int cnt = 0;  // records in the queue
+
+        uint4 vox[NL];
+        // loads of the group whose records start at record i
+        auto issue = [&](int i) {
+            const T* rec = queue + (i + l4) * kRecWords;
+            const unsigned off = __float_as_uint(rec[6]) + 16u * l16;
+            const int span = __float_as_int(rec[3]) & 255;
+            // voxels past the range are not fetched (an offset past the volume reads zeros)
+#pragma unroll
+            for (int k = 0; k < NL; ++k)
+                vox[k] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                       rs, (int)(4 * l16 + 64 * k <= span ? off + 256u * k : 0xfffffff0u), 0, 0));
+        };
+        // the groups of records [0, 4 n)
+        auto drain = [&](auto k_, int n) {
+            constexpr int K = decltype(k_)::value;
+            issue(0);
+            for (int i = 0; i < n; ++i) {
+                const T* rec = queue + (4 * i + l4) * kRecWords;
+                const float4 ra = *(const float4*)rec;
+                const float2 rb = *(const float2*)(rec + 4);
+                const T zinc = ra.x, rz = ra.y, vst = ra.z;
+                const int meta = __float_as_int(ra.w);  // span | first tile cell << 8 | cells << 16
+                const int span = meta & 255;
+                const unsigned cell = (unsigned)(l16 - ((meta >> 8) & 255));
+                // weight of this lane's cell
+                T w = T(0);
+                if (cell < 4u) w = rec[8 + cell];
+                // voxels times sqrt(r^2 + zc^2) to LDS, zeros after the range
+                T zk = rb.y + zl;
+#pragma unroll
+                for (int k = 0; k < NL; ++k) {
+                    float4 o;
+                    T zc = zk;
+                    o.x = fsqrt(fmaf(zc, zc, rb.x)) * __uint_as_float(vox[k].x);
+                    zc += g.dz;
+                    o.y = fsqrt(fmaf(zc, zc, rb.x)) * __uint_as_float(vox[k].y);
+                    zc += g.dz;
+                    o.z = fsqrt(fmaf(zc, zc, rb.x)) * __uint_as_float(vox[k].z);
+                    zc += g.dz;
+                    o.w = fsqrt(fmaf(zc, zc, rb.x)) * __uint_as_float(vox[k].w);
+                    *(float4*)(stage + 64 * k + 4 * l16) = o;
+                    zk += dz64;
+                }
+                if (l16 < 5) stage[span + 1 + l16] = T(0);
+                __builtin_amdgcn_wave_barrier();
+                if (i + 1 < n) issue(4 * i + 4);
+                const T jhi = T(span + 1);
+                T tt = frow - vst;
+#pragma unroll
+                for (int t = 0; t < RT; ++t) {
+                    const T q = careful ? mat_gather_each(stage, jhi, tt, rz, zinc) : mat_gather<K>(stage, jhi, tt, rz, zinc);
+                    tt += T(16);
+                    if constexpr (!careful) {
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, q, acc[t], 0, 0, 0);
+                    } else {
+                        // the footprint's own cells only, zero weights among them included
+                        const int mine = cell < (unsigned)(meta >> 16);
+#pragma unroll 1
+                        for (int k = 0; k < 4; ++k) {
+                            const T qk = __shfl(q, 16 * k + l16, kWave);
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                const T wk = __shfl(w, 16 * k + 4 * l4 + r, kWave);
+                                const int in = __shfl(mine, 16 * k + 4 * l4 + r, kWave);
+                                acc[t][r] = in ? fmaf(wk, qk, acc[t][r]) : acc[t][r];
+                            }
+                        }
+                    }
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+        };
+        int kmax = 2;       // gather class so far: voxels that a row can meet
+
+        // the SPLIT waves of a block take every SPLIT-th image line of the strip
+        for (int m0 = 0; m0 < m_end; m0 += SPLIT * kWave) {
+            const int m = m0 + lane * SPLIT + share;
+            int lo = 0, hi = -1;
+            if (m < m_end) {
+                if (!strip_range(g, v, row_major, m, kL, kR, exhaustive != 0, lo, hi)) hi = lo - 1;
+            }
+            const int lines = hi - lo + 1 > 0 ? hi - lo + 1 : 0;
+            const int incl = wave_incl_scan(lines);
+            const int excl = incl - lines;
+            const int total = rdl_i(incl, kWave - 1);
+            // 64 candidates at a time; where one of them needs more than one record, those 64 again in
+            // four batches of 16 (of at most four records each), so that the queue holds any batch
+            int nb = kWave;
+            for (int k0 = 0; k0 < total;) {
+                const int k = k0 + lane;
+                int j = 0;
+#pragma unroll
+                for (int step = 32; step >= 1; step >>= 1) {
+                    const int e = __shfl(excl, j + step, 64);
+                    if (e <= k) j += step;
+                }
+                const int lo_j = __shfl(lo, j, 64);
+                const int ex_j = __shfl(excl, j, 64);
+                const int minor = lo_j + (k - ex_j);
+                const int ix = row_major ? minor : m0 + j * SPLIT + share;
+                const int iy = row_major ? m0 + j * SPLIT + share : minor;
+                bool ok = k < total && lane < nb;
+                int in_map = 1;
+                if (ok && map != nullptr) in_map = map[iy * g.nx + ix];
+                float4 ra, rb;
+                ColFoot<FOOT> f;
+                T thick = T(14);
+                int c0 = 0, cells = 0, parts = 1;  // a record for every four tile cells of the footprint
+                if (ok) {
+                    const T xc = (T(ix) + g.wx) * g.dx, yc = (T(iy) + g.wy) * g.dy;
+                    int iz0 = 0, iz1 = 0;
+                    ok = col_foot<FOOT>(g, v, xc, yc, f);
+                    ok = ok && f.ihi >= iu_a && f.ilo <= iu_b;
+                    T zinc = T(1), vstart = T(0), rz = T(1);
+                    if (ok) ok = v_window(g, f.d, v.wz, zinc, vstart, iz0, iz1) && iz0 < iz1 && zinc > T(0);
+                    int za = 0, zb = -1;
+                    if (ok) {
+                        // voxel range needed by this item's rows (exact ranges; a voxel left out at
+                        // the rounding edge has a weight of the order of the rounding)
+                        rz = frcp(zinc);
+                        za = max((int)ceil((T(iv_a) - T(0.5) - vstart) * rz - T(1)), iz0);
+                        zb = min((int)ceil((T(iv_last) + T(0.5) - vstart) * rz) - 1, iz1 - 1);
+                        zb = min(zb, za + NV - 1);
+                        ok = za <= zb;
+                    }
+                    if (ok) {
+                        c0 = max(f.ilo, iu_a);
+                        cells = min(f.ihi, iu_b) - c0 + 1;
+                        parts = (cells + 3) >> 2;
+                        ra.x = zinc;
+                        ra.y = rz;
+                        ra.z = vstart + T(za) * zinc;  // lower edge of voxel za
+                        ra.w = __int_as_float((zb - za) | ((c0 - iu_a) << 8) | (min(cells, 4) << 16));
+                        rb.x = f.r2;
+                        rb.y = T(za) * g.dz + wzdz;
+                        rb.z = __uint_as_float(((unsigned)(iy * g.nx + ix) * (unsigned)g.nz + (unsigned)za) * 4u);
+                        rb.w = T(0);
+                        thick = zinc;
+                    }
+                }
+                ok = ok && in_map != 0;
+                if (!ok) parts = 0;
+                const bool wide = __any(parts > 1);
+                if (wide && nb == kWave) {
+                    nb = 16;
+                    continue;
+                }
+                // records in lane order
+                int at, add;
+                if (!wide) {
+                    const unsigned long long mask = __ballot(ok);
+                    at = __popcll(mask & ((1ull << lane) - 1ull));
+                    add = __popcll(mask);
+                } else {
+                    const int inc = wave_incl_scan(parts);
+                    at = inc - parts;
+                    add = rdl_i(inc, kWave - 1);
+                }
+                kmax = max(kmax, __any(thick < T(1) / T(3)) ? 5 : __any(thick < T(0.5)) ? 4 : __any(thick < T(1)) ? 3 : 2);
+                if (ok) {
+                    float4* rec = (float4*)(queue + (cnt + at) * kRecWords);
+                    rec[0] = ra;
+                    rec[1] = rb;
+                    rec[2] = foot_weights<FOOT>(f, c0);
+                    for (int q = 1; q < parts; ++q) {
+                        rec += kRecWords / 4;
+                        rec[0] = make_float4(ra.x, ra.y, ra.z,
+                                             __int_as_float((__float_as_int(ra.w) & 0xffff) + (q << 10) + (min(cells - 4 * q, 4) << 16)));
+                        rec[1] = rb;
+                        rec[2] = foot_weights<FOOT>(f, c0 + 4 * q);
+                    }
+                }
+                cnt += add;
+                k0 += nb;
+                if ((k0 & (kWave - 1)) == 0) nb = kWave;
+                __builtin_amdgcn_wave_barrier();
+                const int n = cnt >> 2;
+                if (n == 0) continue;
+                if (careful || kmax == 5) drain(std::integral_constant<int, 5>{}, n);
+                else if (kmax == 3) drain(std::integral_constant<int, 3>{}, n);
+                else if (kmax == 2) drain(std::integral_constant<int, 2>{}, n);
+                else drain(std::integral_constant<int, 4>{}, n);
+                // the records left over move to the front
+                cnt &= 3;
+                if (lane < cnt * kRecWords) {
+                    const T x = queue[4 * n * kRecWords + lane];
+                    queue[lane] = x;
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+        if (cnt > 0) {
+            // the last group, filled up with columns of zero weight past the volume (zeros)
+            if (lane < 4 - cnt) {
+                float4* rec = (float4*)(queue + (cnt + lane) * kRecWords);
+                rec[0] = make_float4(1.f, 1.f, 0.f, 0.f);
+                rec[1] = make_float4(1.f, 0.f, __uint_as_float(vol_bytes), 0.f);
+                rec[2] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+            __builtin_amdgcn_wave_barrier();
+            drain(std::integral_constant<int, 5>{}, 1);
+        }
+    };
+    walk(std::false_type{});
+    bool finite = true;
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) finite = finite && __builtin_isfinite(acc[t][r]);
+    if (__any(!finite)) walk(std::true_type{});
+
+    // lane l holds cells 4 (l / 16) .. + 3 of row 16 t + l % 16
+    Tout* out = proj + (size_t)b * g.nu * g.nv;
+    if constexpr (SPLIT == 1) {
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const int iv = iv_a + 16 * t + l16;
+            if (iv > iv_last) continue;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int iu = iu_a + 4 * l4 + r;
+                if (iu < g.nu) out[(size_t)iu * g.nv + iv] = cvt_store<Tout>(acc[t][r]);
+            }
+        }
+    } else {
+        // the shares' tiles to LDS; each wave adds its cells in share order and stores them
+        __syncthreads();
+        T* const mine = lds + wv * (TU * kCellW);
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mine[(4 * l4 + r) * kCellW + 16 * t + l16] = acc[t][r];
+        __syncthreads();
+        for (int i = wv; i < TU * RPL; i += WPB) {
+            const int cell = i / RPL, row = (i % RPL) * kWave + lane;
+            T sum = T(0);
+#pragma unroll
+            for (int w = 0; w < WPB; ++w) sum += lds[w * (TU * kCellW) + cell * kCellW + row];
+            if (iu_a + cell < g.nu && iv_a + row <= iv_last)
+                out[(size_t)(iu_a + cell) * g.nv + iv_a + row] = cvt_store<Tout>(sum);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------
 // Matched backprojection: one wavefront per image column, NZL voxels per lane (z
 // fastest).  The views' footprints of the column are evaluated 64 or 32 at a time (one view
 // per lane) into LDS.  Per view the wave then combines the footprint's detector columns
@@ -1823,6 +2257,20 @@ constexpr int kTU2 = 8;  // the same for the two-row-chunk ring form
 // (at most 256); six entries keep five columns in flight in the LDS the FP32 form's four take
 constexpr int kHalfRing1 = 6, kHalfRing2 = 4;
 
+// voxels of a column that the matrix form stages for an item of `rows` detector rows, 0 where
+// it does not cover the geometry: a voxel's height on the detector is zk / d rows, d between
+// the nearest and the farthest column's distance; the volume is addressed with 32-bit offsets
+static int mat_voxels(const Geom<float>& g, int rows) {
+    const double hx = std::max(std::fabs((double)g.wx), std::fabs((double)g.wx + g.nx - 1)) * std::fabs((double)g.dx);
+    const double hy = std::max(std::fabs((double)g.wy), std::fabs((double)g.wy + g.ny - 1)) * std::fabs((double)g.dy);
+    const double R = std::sqrt(hx * hx + hy * hy);
+    if (!(g.sad > R * 1.001 && g.zk > 0.f) || (double)g.nx * g.ny * g.nz * 4.0 > 4.2e9) return 0;
+    const double zmin = g.zk / (g.sad + R) * 0.999, zmax = g.zk / (g.sad - R) * 1.001;
+    if (!(zmin > 0.25 && zmax < 14.0)) return 0;
+    const int need = std::min(g.nz, (int)(rows / zmin) + 4);
+    return need <= 128 ? need : 0;
+}
+
 template <class Tin, class Tout, class T, int FOOT, int RPL, int SPLIT>
 static void launch_proj(unsigned blocks, hipStream_t st, const Geom<T>& g, const View<T>* views, int vstride,
                         int nviews, const void* vol, const uint8_t* map, void* proj, int exhaustive) {
@@ -1842,6 +2290,29 @@ static void launch_proj(unsigned blocks, hipStream_t st, const Geom<T>& g, const
                                dim3(kRW * kWave), 0, st, g, views, vstride, nviews, (const __half*)vol, map,
                                (Tout*)proj, exhaustive);
             return;
+        }
+    }
+    // the matrix form wherever it covers the geometry and the schedule does not ask for the
+    // register pipeline; RPL and the grid come from proj3_foot (form 3: two row chunks per item)
+    if constexpr (std::is_same<Tin, float>::value && std::is_same<T, float>::value) if (form != 2) {
+        const int rows = form == 3 ? 2 * kWave : kWave, need = mat_voxels(g, rows);
+        if (need > 0) {
+            constexpr int kMW = SPLIT > 1 ? 8 : kWavesPerBlock, kMS = SPLIT > 1 ? 8 : 1;
+            const unsigned bytes = (unsigned)((unsigned long long)g.nx * g.ny * g.nz * 4);
+#define CT_MAT(R, NV)                                                                                                  \
+    hipLaunchKernelGGL((cbct_proj_mat_kernel<Tout, FOOT, kMS, R, NV, kMW>), dim3(blocks), dim3(kMW * kWave), 0, st, g, \
+                       views, vstride, nviews, (const float*)vol, bytes, map, (Tout*)proj, exhaustive)
+            if constexpr (SPLIT == 1) {
+                if (form == 3) {
+                    if (need <= 64) CT_MAT(2, 64);
+                    else CT_MAT(2, 128);
+                    return;
+                }
+            }
+            if (need <= 64) CT_MAT(1, 64);
+            else CT_MAT(1, 128);
+            return;
+#undef CT_MAT
         }
     }
     // form 3 (FP32 volumes of at most 256 slices, one wave per item): the ring form with two
@@ -1903,7 +2374,10 @@ static void proj3_foot(const Geom<T>& g, const View<T>* views, int vstride, int 
     const long long items1 = (long long)nviews * ((g.nu + kTU - 1) / kTU) * ((g.nv + kWave - 1) / kWave);
     const bool two = fp32 && g.nz <= 4 * kWave &&
                      (form == 3 || (form == 0 && ssplit0 != 2 && g.nv > kWave && items1 >= 16384));
-    const int tu = two ? kTU2 : kTU, rows = two ? 2 * kWave : kWave;
+    int tu = two ? kTU2 : kTU;
+    if constexpr (fp32)
+        if (two && mat_voxels(g, 2 * kWave) > 0) tu = kTU;  // the matrix form keeps 16-cell tiles
+    const int rows = two ? 2 * kWave : kWave;
     const long long nut = (g.nu + tu - 1) / tu, nvc = (g.nv + rows - 1) / rows;
     const long long items = (long long)nviews * nut * nvc;
     if (two) {

@@ -186,10 +186,11 @@ int ctsim_plan_create(ctsim_plan** plan, int32_t ndim, const ctsim_geom* g, int3
 int ctsim_plan_destroy(ctsim_plan* plan);
 /* Launch schedules of a 3D plan (no counterpart in the reference, whose CUDA path uses
  * fixed 16 x 16 blocks, geom/dd_cuda/cbct_dd_proj.c:441-442).  proj_sched = form | split << 2:
- * form 0 automatic, 1 LDS-ring forward kernel (FP32 volumes of at most 256 slices, FP16
- * volumes of an even number of at most 256), 2 register-pipeline forward kernel, 3 the ring
- * kernel with two 64-row chunks per item and eight-cell tiles (FP32 volumes of at most 256
- * slices, one wave per item; others take the automatic form); split 0
+ * form 0 automatic, 1 the matrix forward kernel (FP32 volumes whose voxels are 1/4 to
+ * 14 detector rows thick) or the LDS-ring one (other FP32 volumes of at most 256 slices, FP16
+ * volumes of an even number of at most 256), 2 register-pipeline forward kernel, 3 the same
+ * with two 64-row chunks per item (FP32 volumes in the matrix kernel's range, or of at most 256
+ * slices; one wave per item; others take the automatic form); split 0
  * automatic (a block's waves share a work item below 16384 items), 1 one wave per item,
  * 2 shared items.  back_sched bit 0 (DD / SF backprojection): 0 four consecutive image
  * columns per block, 1 2 x 2 column patches in 32 x 32 super-tiles (both with a contiguous
