@@ -1822,6 +1822,256 @@ __global__ __launch_bounds__(kBlock) void cbct_back_kernel(Geom<T> g, const View
 }
 
 // ---------------------------------------------------------------------------------
+// Matched backprojection, four columns per wave (FP32 arithmetic, voxels of at most three rows,
+// detectors of at most kQuadRows rows).  The same footprints, u combination and row gathers as
+// cbct_back_kernel; what differs is that a view is handled for a 2 x 2 patch of columns at a
+// time, 16 lanes to a column, so that the chain of a view (its record, its rows, their
+// combination in LDS, the gathers) is waited for once per four columns:
+//
+//  * footprints of 16 views x 4 columns are evaluated one per lane;
+//  * a lane loads four rows of each footprint cell at once (8 or 16 bytes; one load per cell and
+//    64 rows of four columns, where the one-column form takes one per cell and column), combines
+//    them and writes them to its column's row buffer, words of rows past the detector as zeros;
+//  * the next view's first rows load while this one is gathered;
+//  * lane l % 16 owns voxels l % 16 + 16 i of its column, all parameters in vector registers.
+//
+// Latency bounds it, as it does the one-column form (which ran no faster with its footprint
+// arithmetic cut by a fifth): three blocks of four waves per CU where the column's 32 voxels per
+// lane need the registers (at four they spill: 512-slice columns 3.95 ms against 2.16), else
+// four (six spill FP32: 62.5 ms against 51.9 below).  Against the one-column form: SF of 512^2 x
+// 64 from a subset of 82 BF16 views 0.94 -> 0.80 ms; DD of 512^2 x 256 from 720 FP32 views
+// 82.6 -> 51.9 ms; DD of 256^2 x 512 from 60 views 3.09 -> 2.16 ms.
+// ---------------------------------------------------------------------------------
+constexpr int kQuadRows = 768;  // four row buffers per wave within 64 KB of LDS per block
+constexpr int kQuadViews = 16, kQuadRec = 14;  // views per batch, words per record
+constexpr int kQuadCells = 8;                  // footprint cells a record holds weights for
+// words of one column's row buffer: four zeros, the rows in 64-row chunks, eight zeros (a gather that
+// starts at either end meets zeros only, whatever rows an earlier view left)
+__host__ __device__ inline int quad_pitch(int nv) { return 4 + (nv + kWave - 1) / kWave * kWave + 8; }
+inline size_t quad_lds(int nv) { return (size_t)kWavesPerBlock * (4 * quad_pitch(nv) + kWave * kQuadRec) * sizeof(float); }
+
+// four consecutive rows at a byte offset, as floats
+template <class Tin>
+struct Rows4 {
+    typename std::conditional<sizeof(Tin) == 4, uint4, uint2>::type x;
+};
+template <class Tin>
+__device__ __forceinline__ Rows4<Tin> load_rows4(__amdgpu_buffer_rsrc_t rs, unsigned off) {
+    Rows4<Tin> r;
+    if constexpr (sizeof(Tin) == 4) r.x = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
+    else r.x = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rs, (int)off, 0, 0));
+    return r;
+}
+template <class Tin>
+__device__ __forceinline__ float4 rows4_f(const Rows4<Tin>& r) {
+    if constexpr (sizeof(Tin) == 4) {
+        return __builtin_bit_cast(float4, r.x);
+    } else {
+        auto f = [](unsigned h) {
+            const unsigned short b = (unsigned short)h;
+            return to_f(__builtin_bit_cast(Tin, b));
+        };
+        return make_float4(f(r.x.x & 0xffffu), f(r.x.x >> 16), f(r.x.y & 0xffffu), f(r.x.y >> 16));
+    }
+}
+
+template <class Tin, class Tout, int FOOT, int NZ>
+__global__ __launch_bounds__(kBlock, NZ >= 32 ? 3 : 4) void cbct_back_quad_kernel(Geom<float> g, const View<float>* __restrict__ views,
+                                                                int vstride, int nviews, const Tin* __restrict__ proj,
+                                                                const uint8_t* __restrict__ map,
+                                                                Tout* __restrict__ vol, float scale, int accumulate) {
+    using T = float;
+    extern __shared__ __align__(16) unsigned char back_dyn_lds[];
+    const int wv = (int)(threadIdx.x / kWave), lane = lane_id(), l16 = lane & 15, l4 = lane >> 4;
+    const int pitch = quad_pitch(g.nv);
+    T* const wave = reinterpret_cast<T*>(back_dyn_lds) + wv * (4 * pitch + kWave * kQuadRec);
+    // records as arrays over 16 views x 4 columns: (thickness, start, r^2, z), weights, more weights, (offset, rows)
+    float4* const recs = (float4*)(wave + 4 * pitch);
+    int2* const recx = (int2*)(recs + 3 * kWave);
+    T* const sw = wave + l4 * pitch;  // rows at sw[4 + row]
+    // column order (g.sched_back bit 0): 0 = sixteen consecutive columns per block; 1 = 4 x 4
+    // columns (2 x 2 per wave) in super-tiles of kSuperTile x kSuperTile
+    constexpr int kB = kSuperTile / 4;
+    constexpr bool kAhead = NZ >= 16;  // tall columns: registers for the next 64 rows' loads
+    int ix, iy;
+    if (g.sched_back & 1) {
+        const int stl = blockIdx.x / (kB * kB), r = blockIdx.x % (kB * kB);
+        const int stx = (g.nx + kSuperTile - 1) / kSuperTile;
+        ix = (stl % stx) * kSuperTile + (r % kB) * 4 + (wv & 1) * 2 + (l4 & 1);
+        iy = (stl / stx) * kSuperTile + (r / kB) * 4 + (wv >> 1) * 2 + (l4 >> 1);
+    } else {
+        const int col = (blockIdx.x * kWavesPerBlock + wv) * 4 + l4;
+        iy = col / g.nx;
+        ix = col - iy * g.nx;
+    }
+    const bool inside = ix < g.nx && iy < g.ny;
+    const bool active = inside && (map == nullptr || map[iy * g.nx + ix] != 0);
+    T img[NZ];
+#pragma unroll
+    for (int i = 0; i < NZ; ++i) img[i] = T(0);
+    if (__any(active)) {
+        for (int i = lane; i < 4 * pitch; i += kWave) wave[i] = T(0);
+        const T xc = (T(ix) + g.wx) * g.dx, yc = (T(iy) + g.wy) * g.dy;
+        const T fz = T(l16), zd = T(l16) * g.dz, dz16 = T(16) * g.dz;
+        const T fhi = T(g.nv + 4);
+        const int row0 = 4 * l16, cellb = g.nv * (int)sizeof(Tin);
+        const size_t view_elems = (size_t)g.nu * g.nv;
+        for (int b0 = 0; b0 < nviews; b0 += kQuadViews) {
+            const int nb = min(kQuadViews, nviews - b0);
+            // footprint of view b0 + l16 on this lane's column; columns that the view misses get
+            // zero weights and no cells
+            {
+                float4* rec = recs + l16 * 4 + l4;
+                bool ok = active && l16 < nb;
+                // (no thickness, past the last row: where the gathers read the zeros at the end)
+                float4 ra = make_float4(0.f, 2048.f, 0.f, 0.f), rw = make_float4(0.f, 0.f, 0.f, 0.f), rx = rw;
+                int voff = 0, rows = 0x3ff;  // rows r0 | r1 << 10, empty: r0 above r1; cells << 20
+                if (ok) {
+                    const View<T> v = views[(size_t)(b0 + l16) * vstride];
+                    ColFoot<FOOT> f;
+                    ok = col_foot<FOOT>(g, v, xc, yc, f);
+                    T zinc = T(1), vstart = T(0);
+                    int iz0 = 0, iz1 = 0;
+                    const T wz = v.wz + g.zoff;
+                    if (ok) ok = v_window(g, f.d, wz, zinc, vstart, iz0, iz1) && iz0 < iz1 && zinc > T(0);
+                    if (ok) {
+                        // rows touched by voxels iz0 .. iz1 - 1
+                        const T a0 = fmaxf(vstart + T(iz0) * zinc + T(0.5), T(0));
+                        const T a1 = fminf(vstart + T(iz1 - 1) * zinc + zinc + T(0.5), T(g.nv));
+                        ok = a0 <= a1;
+                        if (ok) {
+                            const int cells = f.ihi - f.ilo + 1;
+                            rows = min((int)floor(a0), g.nv - 1) | (min((int)floor(a1), g.nv - 1) << 10) | (cells << 20);
+                            ra = make_float4(zinc, vstart + T(4.5), f.r2, wz * g.dz);
+                            rw = foot_weights<FOOT>(f, f.ilo);
+                            if (cells > 4) rx = foot_weights<FOOT>(f, f.ilo + 4);
+                            voff = (int)(((unsigned)(l16 * g.nu + f.ilo) * (unsigned)g.nv) * (unsigned)sizeof(Tin));
+                        }
+                    }
+                }
+                rec[0] = ra;
+                rec[64] = rw;
+                rec[128] = rx;
+                recx[l16 * 4 + l4] = make_int2(voff, rows);
+            }
+            __builtin_amdgcn_wave_barrier();
+            const auto rs = buf_rsrc(proj + (size_t)b0 * view_elems, (int)((unsigned)nb * (unsigned)view_elems * (unsigned)sizeof(Tin)));
+            Rows4<Tin> pre[4];
+            int first = 0, last = -1;  // row chunks that the view's columns reach
+            // cells past the footprint's last are not fetched (an offset past the views reads zeros)
+            auto load4 = [&](unsigned off, int n, Rows4<Tin>* out) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) out[k] = load_rows4<Tin>(rs, k < n ? off + (unsigned)(k * cellb) : 0xfffffff0u);
+            };
+            auto begin = [&](int k) {
+                const int2 rc = recx[k * 4 + l4];
+                const int r0 = rc.y & 0x3ff, r1 = (rc.y >> 10) & 0x3ff;
+                first = 0x3fff;
+                last = -1;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const int a = rdl_i(r0, 16 * c), b = rdl_i(r1, 16 * c);
+                    if (a <= b) {
+                        first = min(first, a);
+                        last = max(last, b);
+                    }
+                }
+                if (last < 0) return;
+                first >>= 6;
+                last = min((last + kRowPad) >> 6, (g.nv - 1) >> 6);
+                load4((unsigned)rc.x + (unsigned)((64 * first + row0) * (int)sizeof(Tin)), rc.y >> 20, pre);
+            };
+            begin(0);
+            for (int k = 0; k < nb; ++k) {
+                const float4* rec = recs + k * 4 + l4;
+                const int c0 = first, c1 = last;
+                if (c1 < 0) {
+                    if (k + 1 < nb) begin(k + 1);
+                    continue;
+                }
+                const float4 w = rec[64];
+                const int2 rc = recx[k * 4 + l4];
+                const int cells = rc.y >> 20;
+                const bool wide = __any(cells > 4);
+                // u combination, 64 rows of the four columns at a time
+                for (int c = c0; c <= c1; ++c) {
+                    const unsigned off = (unsigned)rc.x + (unsigned)((64 * c + row0) * (int)sizeof(Tin));
+                    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+                    auto add = [&](const float4& wk, const Rows4<Tin>* x) {
+                        const float wq[4] = {wk.x, wk.y, wk.z, wk.w};
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const float4 p = rows4_f(x[q]);
+                            o.x = fmaf(wq[q], p.x, o.x);
+                            o.y = fmaf(wq[q], p.y, o.y);
+                            o.z = fmaf(wq[q], p.z, o.z);
+                            o.w = fmaf(wq[q], p.w, o.w);
+                        }
+                    };
+                    auto more = [&](Rows4<Tin>* x) {  // a footprint of more than four cells
+                        load4(off + (unsigned)(4 * cellb), cells - 4, x);
+                        add(rec[128], x);
+                    };
+                    const unsigned next = off + 64u * (unsigned)sizeof(Tin);
+                    if constexpr (kAhead) {
+                        Rows4<Tin> cur[4];
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) cur[q] = pre[q];
+                        if (c < c1) load4(next, cells, pre);
+                        add(w, cur);
+                        if (wide) more(cur);
+                    } else {
+                        add(w, pre);
+                        if (wide) more(pre);
+                        if (c < c1) load4(next, cells, pre);
+                    }
+                    const int left = g.nv - 64 * c - row0;  // rows of the detector from this lane's first on
+                    o.x = left > 0 ? o.x : T(0);
+                    o.y = left > 1 ? o.y : T(0);
+                    o.z = left > 2 ? o.z : T(0);
+                    o.w = left > 3 ? o.w : T(0);
+                    *(float4*)(sw + 4 + 64 * c + row0) = o;
+                }
+                __builtin_amdgcn_wave_barrier();
+                if (k + 1 < nb) begin(k + 1);
+                const float4 ra = rec[0];
+                const T zinc = ra.x, r2 = ra.z;
+                // the group's class: rows that its thickest voxels meet
+                auto voxels = [&](auto k_) {
+                    constexpr int K = decltype(k_)::value;
+                    const T zm1 = zinc - T(1);
+                    T fi = fz, zc = zd + ra.w;
+#pragma unroll
+                    for (int i = 0; i < NZ; ++i) {
+                        const T a = fmaf(fi, zinc, ra.y);
+                        T s;
+                        if constexpr (K == 2) s = gather_rows2<T>(sw, T(0), fhi, a, zinc, zm1);
+                        else s = gather_rows<T, K>(sw, T(0), fhi, a, a + zinc);
+                        img[i] = fmaf(fsqrt(fmaf(zc, zc, r2)), s, img[i]);
+                        fi += T(16);
+                        zc += dz16;
+                    }
+                };
+                if (!__any(zinc > T(1))) voxels(std::integral_constant<int, 2>{});
+                else if (!__any(zinc > T(2))) voxels(std::integral_constant<int, 3>{});
+                else voxels(std::integral_constant<int, 4>{});
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+    }
+    if (!inside) return;
+    Tout* ocol = vol + (size_t)(iy * g.nx + ix) * g.zstride;
+#pragma unroll
+    for (int i = 0; i < NZ; ++i) {
+        const int iz = 16 * i + l16;
+        if (iz < g.nz) {
+            const T val = scale * img[i];
+            ocol[iz] = cvt_store<Tout>(accumulate ? ld<T>(ocol + iz) + val : val);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------
 // FDK voxel-driven bilinear backprojection (cbct_back1_pd).  off_boundary = 1 is
 // 'back,pd' (skip below the detector, stop above it), 0 is 'back,hpd' (clamp v).
 // One wavefront per image column, NZL voxels per lane.
@@ -2451,6 +2701,46 @@ static void launch_back_dd_tf(unsigned blocks, hipStream_t st, const Geom<T>& g,
                            (Tout*)vol, scale, accumulate, rowwin, NestArgs{}, g.sched_back & 1);
 }
 
+// whether the four-column form takes a backprojection: FP32, voxels of at most three rows at
+// the nearest column, footprints of at most kQuadCells cells, rows addressed in whole words,
+// and enough columns that a quarter of the waves still fills the chip:
+// below that the one-column form's larger number of waves wins (64 slices: 64^2 columns 45 us
+// against 69, 112^2 98 against 101, 256^2 345 against 292; 256 slices: 64^2 146 against 167,
+// 80^2 245 against 211, 128^2 421 against 268)
+template <class Tin, class T, int NZL>
+static bool quad_ok(const Geom<T>& g, const void* proj) {
+    if constexpr (sizeof(T) != 4) return false;
+    if (g.nv > kQuadRows) return false;
+    if ((long long)g.nx * g.ny < (NZL == 1 ? 16384 : 6400)) return false;
+    if ((g.nv * sizeof(Tin)) % 4 != 0 || (uintptr_t)proj % 4 != 0) return false;
+    const double hx = std::max(std::fabs((double)g.wx), std::fabs((double)g.wx + g.nx - 1)) * std::fabs((double)g.dx);
+    const double hy = std::max(std::fabs((double)g.wy), std::fabs((double)g.wy + g.ny - 1)) * std::fabs((double)g.dy);
+    const double R = std::sqrt(hx * hx + hy * hy);
+    if (!(g.zk > 0 && g.sad > R * 1.001 && g.zk / (g.sad - R) * 1.001 <= 3.0)) return false;
+    // footprint width in cells: the pixel's angle from the source, times the cells per radian at
+    // the edge of the image on a flat detector; a width of w meets at most w + 2 cells
+    const double h = 0.5 * std::sqrt((double)g.dx * g.dx + (double)g.dy * g.dy), near_ = g.sad - R - h;
+    if (!(near_ > 2.0 * h)) return false;
+    const double c2 = 1.0 - (R + h) * (R + h) / ((double)g.sad * g.sad);
+    return c2 > 0.0 && 2.0 * std::asin(h / near_) * std::fabs((double)g.sdd_du) / c2 + 2.0 <= kQuadCells;
+}
+
+template <class Tin, class Tout, class T, int NZL>
+static void launch_back_quad(hipStream_t st, const Geom<T>& g, const View<T>* views, int vstride, int nviews,
+                             const void* proj, const uint8_t* map, void* vol, int foot, T scale, int accumulate) {
+    if constexpr (sizeof(T) == 4) {
+        const int tiles = ((g.nx + kSuperTile - 1) / kSuperTile) * ((g.ny + kSuperTile - 1) / kSuperTile);
+        const unsigned blocks = (g.sched_back & 1) ? (unsigned)(tiles * (kSuperTile * kSuperTile / 16))
+                                                   : (unsigned)(((long long)g.nx * g.ny + 15) / 16);
+#define CT_QUAD(F)                                                                                                  \
+    hipLaunchKernelGGL((cbct_back_quad_kernel<Tin, Tout, F, 4 * NZL>), dim3(blocks), dim3(kBlock), quad_lds(g.nv), st, \
+                       g, views, vstride, nviews, (const Tin*)proj, map, (Tout*)vol, scale, accumulate)
+        if (foot == FOOT_DD) CT_QUAD(FOOT_DD);
+        else CT_QUAD(FOOT_TF);
+#undef CT_QUAD
+    }
+}
+
 template <class Tin, class Tout, class T, int NZL>
 static void launch_back(unsigned blocks, hipStream_t st, const Geom<T>& g, const View<T>* views, int vstride,
                         int nviews, const void* proj, const uint8_t* map, void* vol, int foot, int pd_mode, T scale,
@@ -2478,6 +2768,8 @@ static void launch_back(unsigned blocks, hipStream_t st, const Geom<T>& g, const
         hipLaunchKernelGGL((cbct_back_pd_kernel<Tin, Tout, T, NZL, 0>), dim3(blocks), dim3(kBlock), 0, st, g, views,
                            vstride, nviews, (const Tin*)proj, map, (Tout*)vol, scale, accumulate,
                            pd_limits<T>(g.nu, g.nv));
+    else if (quad_ok<Tin, T, NZL>(g, proj))
+        launch_back_quad<Tin, Tout, T, NZL>(st, g, views, vstride, nviews, proj, map, vol, foot, scale, accumulate);
     else if (g.nv <= kWave)
         launch_back_dd_tf<Tin, Tout, T, NZL, true>(blocks, st, g, views, vstride, nviews, proj, map, vol, foot, scale,
                                                    accumulate, rowwin);

@@ -192,9 +192,8 @@ int ctsim_plan_destroy(ctsim_plan* plan);
  * with two 64-row chunks per item (FP32 volumes in the matrix kernel's range, or of at most 256
  * slices; one wave per item; others take the automatic form); split 0
  * automatic (a block's waves share a work item below 16384 items), 1 one wave per item,
- * 2 shared items.  back_sched bit 0 (DD / SF backprojection): 0 four consecutive image
- * columns per block, 1 2 x 2 column patches in 32 x 32 super-tiles (both with a contiguous
- * range per XCD); bit 1 (FDK pd / hpd, FP32 plans): 0 the LDS-staged form (detectors of at
+ * 2 shared items.  back_sched bit 0 (DD / SF backprojection): 0 consecutive image columns, 1
+ * 2 x 2 column patches in 32 x 32 super-tiles (either way the same terms in the same order); bit 1 (FDK pd / hpd, FP32 plans): 0 the LDS-staged form (detectors of at
  * most 1024 rows; taller ones take the direct form), 1 the direct form.  A new plan has
  * (0, 1).  Every schedule is deterministic; the forward forms and splits, and the two FDK
  * forms, add terms in different orders, so their results agree to FP32 rounding, not bit
