@@ -1839,7 +1839,7 @@ __global__ __launch_bounds__(kBlock) void cbct_back_kernel(Geom<T> g, const View
 // arithmetic cut by a fifth): three blocks of four waves per CU where the column's 32 voxels per
 // lane need the registers (at four they spill: 512-slice columns 3.95 ms against 2.16), else
 // four (six spill FP32: 62.5 ms against 51.9 below).  Against the one-column form: SF of 512^2 x
-// 64 from a subset of 82 BF16 views 0.94 -> 0.80 ms; DD of 512^2 x 256 from 720 FP32 views
+// 128 from a subset of 41 BF16 views 0.93 -> 0.80 ms; DD of 512^2 x 256 from 720 FP32 views
 // 82.6 -> 51.9 ms; DD of 256^2 x 512 from 60 views 3.09 -> 2.16 ms.
 // ---------------------------------------------------------------------------------
 constexpr int kQuadRows = 768;  // four row buffers per wave within 64 KB of LDS per block
@@ -2706,12 +2706,16 @@ static void launch_back_dd_tf(unsigned blocks, hipStream_t st, const Geom<T>& g,
 // and enough columns that a quarter of the waves still fills the chip:
 // below that the one-column form's larger number of waves wins (64 slices: 64^2 columns 45 us
 // against 69, 112^2 98 against 101, 256^2 345 against 292; 256 slices: 64^2 146 against 167,
-// 80^2 245 against 211, 128^2 421 against 268)
+// 80^2 245 against 211, 128^2 421 against 268).  On detectors of at most 64 rows the one-column
+// form keeps a whole column's rows in one pass and its taller columns win unless the image is
+// large (106 x 102 x 142 from 58 rows FP16 124 us against 147, 252 x 197 x 80 FP32 1007 against
+// 1081, 500 x 350 x 143 BF16 744 against 759; but 512^2 x 128 BF16 934 against 803)
 template <class Tin, class T, int NZL>
 static bool quad_ok(const Geom<T>& g, const void* proj) {
     if constexpr (sizeof(T) != 4) return false;
     if (g.nv > kQuadRows) return false;
-    if ((long long)g.nx * g.ny < (NZL == 1 ? 16384 : 6400)) return false;
+    const long long cols = (long long)g.nx * g.ny;
+    if (NZL == 1 ? cols < 16384 : g.nv > kWave ? cols < 6400 : NZL > 2 || sizeof(Tin) != 2 || cols < 65536) return false;
     if ((g.nv * sizeof(Tin)) % 4 != 0 || (uintptr_t)proj % 4 != 0) return false;
     const double hx = std::max(std::fabs((double)g.wx), std::fabs((double)g.wx + g.nx - 1)) * std::fabs((double)g.dx);
     const double hy = std::max(std::fabs((double)g.wy), std::fabs((double)g.wy + g.ny - 1)) * std::fabs((double)g.dy);
