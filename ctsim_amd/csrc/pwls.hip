@@ -162,7 +162,15 @@ __device__ __forceinline__ void finish_reduction(double block_value, RedScratch 
 
 // ---------------------------------------------------------------------------------
 // residual r = w .* (p - y) and phi += sum(w .* (p - y).^2) / 2
+//
+// What bounds it at a subset's size is not the data but the end of the reduction: every block
+// makes its partial sum visible to the other dies and adds to one counter, one block after the
+// other.  So few blocks (res_grid), each thread with the loads of four elements in flight.
+// A subset of 0.54M FP16 elements: 24.5 us with up to 1024 blocks of one element at a time,
+// 9.9 us now.
 // ---------------------------------------------------------------------------------
+constexpr int kResUnroll = 4;   // elements of a thread loaded together
+constexpr int kResBlocks = 512;  // two blocks per CU: 6 MB of FP32 loads in flight
 template <class P, class Y, class W, class R>
 __global__ __launch_bounds__(kRB) void residual_kernel(const P* __restrict__ p, const Y* __restrict__ y,
                                                        const W* __restrict__ w, R* __restrict__ r, size_t n,
@@ -172,12 +180,25 @@ __global__ __launch_bounds__(kRB) void residual_kernel(const P* __restrict__ p, 
                                             std::is_same<W, double>::value,
                                         double, float>::type;
     double acc = 0.0;
-    for (size_t i = (size_t)blockIdx.x * kRB + threadIdx.x; i < n; i += (size_t)gridDim.x * kRB) {
-        const C d = ld<C>(p + i) - ld<C>(y + i);
-        const C wi = ld<C>(w + i);
+    auto one = [&](size_t i, C pi, C yi, C wi) {
+        const C d = pi - yi;
         r[i] = cvt_store<R>(wi * d);
         acc += (double)wi * (double)d * (double)d;
+    };
+    const size_t step = (size_t)gridDim.x * kRB;
+    size_t i = (size_t)blockIdx.x * kRB + threadIdx.x;
+    for (; i + (kResUnroll - 1) * step < n; i += kResUnroll * step) {
+        C pi[kResUnroll], yi[kResUnroll], wi[kResUnroll];
+#pragma unroll
+        for (int k = 0; k < kResUnroll; ++k) {
+            pi[k] = ld<C>(p + i + k * step);
+            yi[k] = ld<C>(y + i + k * step);
+            wi[k] = ld<C>(w + i + k * step);
+        }
+#pragma unroll
+        for (int k = 0; k < kResUnroll; ++k) one(i + k * step, pi[k], yi[k], wi[k]);
     }
+    for (; i < n; i += step) one(i, ld<C>(p + i), ld<C>(y + i), ld<C>(w + i));
     const double bs = block_sum(acc);
     finish_reduction(0.5 * wscale * bs, rs, phi, 1);
 }
@@ -673,10 +694,16 @@ static unsigned red_grid(size_t n) {
     return (unsigned)(b < (size_t)kRedBlocks ? (b == 0 ? 1 : b) : kRedBlocks);
 }
 
+// eight elements per thread up to kResBlocks blocks
+static unsigned res_grid(size_t n) {
+    const size_t b = (n + 8 * kRB - 1) / (8 * kRB);
+    return (unsigned)std::min<size_t>(std::max<size_t>(b, 1), kResBlocks);
+}
+
 template <class P, class Y, class W>
 static hipError_t residual_r(const void* p, const void* y, const void* w, void* r, int rdt, size_t n, double ws,
                              RedScratch rs, double* phi, hipStream_t st) {
-    const unsigned gb = red_grid(n);
+    const unsigned gb = res_grid(n);
     switch (rdt) {
         case DT_F32: hipLaunchKernelGGL((residual_kernel<P, Y, W, float>), dim3(gb), dim3(kRB), 0, st, (const P*)p, (const Y*)y, (const W*)w, (float*)r, n, ws, rs, phi); break;
         case DT_F16: hipLaunchKernelGGL((residual_kernel<P, Y, W, __half>), dim3(gb), dim3(kRB), 0, st, (const P*)p, (const Y*)y, (const W*)w, (__half*)r, n, ws, rs, phi); break;
@@ -712,7 +739,7 @@ static hipError_t residual_launch_rs(const void* p, int pdt, const void* y, int 
                                      int rdt, size_t n, double ws, double* phi, RedScratch rs, hipStream_t st) {
     if (pdt == DT_F64 || ydt == DT_F64 || wdt == DT_F64 || rdt == DT_F64) {
         if (pdt != DT_F64 || ydt != DT_F64 || wdt != DT_F64 || rdt != DT_F64) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((residual_kernel<double, double, double, double>), dim3(red_grid(n)), dim3(kRB), 0, st,
+        hipLaunchKernelGGL((residual_kernel<double, double, double, double>), dim3(res_grid(n)), dim3(kRB), 0, st,
                            (const double*)p, (const double*)y, (const double*)w, (double*)r, n, ws, rs, phi);
         return hipGetLastError();
     }
