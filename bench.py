@@ -216,7 +216,7 @@ def pair_gups(kinds=("dd", "tf"), reps=2):
                          proj_tflops=round(pt, 2), back_tflops=round(bt, 2),
                          proj_frac=round(pt / PEAK_FP32_TFLOPS, 4), back_frac=round(bt / PEAK_FP32_TFLOPS, 4),
                          schedule={"proj": tp_sched, "back": tb_sched,
-                                   "codes": "proj form|split<<2 (form 0 auto, 1 ring, 2 register, 3 ring with two row chunks; split 0 auto, "
+                                   "codes": "proj form|split<<2 (form 0 auto, 1 matrix or ring, 2 register, 3 the same with two row chunks; split 0 auto, "
                                             "1 whole, 2 shared); back 0 linear, 1 super-tile"})
         log(f"pair {kind}: proj {tp:.1f} ms  back {tb:.1f} ms  {out[kind]['gups_pair']} GUPS")
     return out
@@ -541,14 +541,11 @@ def main():
     # dominant kernel: the forward projector (per-subset launch)
     f_launch = flops(c_it) / M
     achieved = f_launch / (kt["proj"] * 1e-3) / 1e12
-    ring = (sched[0] & 3) != 2
-    split = (sched[0] >> 2) & 3
-    kname = ("cbct_proj_ring_kernel<float,SF,16,8,2,8>" if ring and split != 1 else
-             "cbct_proj_ring_kernel<float,SF,16,1,2,4>" if ring else "cbct_proj_kernel<float,float,float,SF,16,1,*>")
+    kname = ("cbct_proj_mat_kernel<float,SF,*>" if (sched[0] & 3) != 2 else "cbct_proj_kernel<float,float,float,SF,16,1,*>")
     roof = dict(bound="valu", achieved=round(achieved, 3), peak=PEAK_FP32_TFLOPS, unit="TFLOP/s",
                 frac=round(achieved / PEAK_FP32_TFLOPS, 4), traffic=measured_traffic(),
                 kernel=f"{kname} (one 41-view subset, FP32 input z - x0, autotuned schedule {sched[0]})",
-                note="FP32 vector ALU bound, no MFMA (not a dense contraction); peak = MI355X's published FP32 "
+                note="footprints and gathers on the FP32 vector ALU, tiles by the FP32 matrix instruction; peak = MI355X's published FP32 "
                      "figure; achieved = (17U+3C+60K)/24 per launch / HIP-event time on the launch stream")
     res = {
         "metric": "PWLS-OS iter/s at 512²×128 and DD proj+backproj GUPS, mixed vs plain FP32",
@@ -575,7 +572,7 @@ def main():
         "kernel_ms_per_subset": {k: round(v, 4) for k, v in kt.items()},
         "autotune": {"schedule": {"proj": sched[0], "back": sched[1]}, "proj": tuning["proj"],
                      "back": tuning["back"],
-                     "codes": "proj form|split<<2 (form 0 auto, 1 ring, 2 register, 3 ring with two row chunks; split 0 auto, 1 whole, "
+                     "codes": "proj form|split<<2 (form 0 auto, 1 matrix or ring, 2 register, 3 the same with two row chunks; split 0 auto, 1 whole, "
                               "2 shared); back 0 linear, 1 super-tile; times in ms per 41-view launch"},
         "roofline": roof,
         "accuracy": accuracy,
