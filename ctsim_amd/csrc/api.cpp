@@ -889,6 +889,7 @@ struct ctsim_batch2 {
     int proj_split = 1;  // waves per forward work item (strip split)
     int back_split = 4;  // waves per backprojection work item (view split)
     int form[2] = {0, 0};  // forward form of DD and SF: 0 candidates, 1 line walk (flat), 2 line walk (arc)
+    int back_skip = 0;     // backprojection: views passed over that no pixel of a wave sees
 };
 
 namespace {
@@ -947,6 +948,7 @@ int batch2_build(ctsim_batch2* b, int n, const ctsim_geom* geoms, const int32_t*
                 ok = ok && fan_walk_ok(sl[i].g, kind) && (sl[i].g.dettype == 1) == (sl[0].g.dettype == 1);
             b->form[kind] = ok ? (sl[0].g.dettype == 1 ? 1 : 2) : 0;
         }
+        for (int i = 0; i < n; ++i) b->back_skip |= fan_back_skips(sl[i].g);
     }
     b->proj_split = ip < kFewItems2D ? 4 : 1;  // the single-slice forward's rule
     b->img_elems = img;
@@ -1021,9 +1023,9 @@ int ctsim_batch2_back(const ctsim_batch2* b, const char* op, const void* d_sino,
     const int kind = k == OP_BACK_DD ? 0 : k == OP_BACK_TF ? 1 : 2;
     hipError_t e = b->compute == CTSIM_F32
                        ? fbct_back_batch_launch<float>(b->d_slices_back, b->nslices, b->nitems_back, d_sino, sino_dt,
-                                                       d_img, img_dt, kind, b->back_split, (hipStream_t)stream)
+                                                       d_img, img_dt, kind, b->back_split, b->back_skip, (hipStream_t)stream)
                        : fbct_back_batch_launch<double>(b->d_slices_back, b->nslices, b->nitems_back, d_sino, sino_dt,
-                                                        d_img, img_dt, kind, b->back_split, (hipStream_t)stream);
+                                                        d_img, img_dt, kind, b->back_split, 0, (hipStream_t)stream);
     if (e == hipErrorInvalidValue) return fail(CTSIM_EUNSUP, "Error: dtype combination not supported.");
     HIP_TRY(e, "batched backprojection");
     return CTSIM_OK;

@@ -100,7 +100,10 @@ hipError_t fbct_proj_batch_launch(const void* slices, int nslices, int nitems, c
 bool fan_walk_ok(const Geom<float>& g, int kind);
 template <class T>
 hipError_t fbct_back_batch_launch(const void* slices, int nslices, int nitems, const void* proj, int proj_dt,
-                                  void* img, int img_dt, int kind, int split, hipStream_t st);
+                                  void* img, int img_dt, int kind, int split, int skip, hipStream_t st);
+// whether the FP32 matched backprojection passes over views that no pixel of a wave sees; a batch
+// takes one kernel for all of its slices, this one where any of them asks for it
+bool fan_back_skips(const Geom<float>& g);
 size_t slice2_size(bool dbl);
 
 // utility kernels

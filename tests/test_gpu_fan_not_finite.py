@@ -18,12 +18,14 @@ FANS = {
     # the image overhangs the detector on both sides, by most of it on the low side
     "overhang": ((60, 50), (1.2, 1.2), 40, 1.0, 14.0, 1000.0, 1500.0, 1),
     "overhang_arc": ((60, 50), (1.2, 1.2), 40, 1.0, 14.0, 600.0, 1100.0, 0),
+    # the same so far that views are passed over (images of 256^2 pixels and more)
+    "far_overhang": ((260, 256), (1.2, 1.2), 40, 1.0, 14.0, 1000.0, 1500.0, 1),
     # pixels of two to four cells, inside the detector; oblong pixels
     "fine_cells": ((31, 44), (1.5, 1.1), 200, 0.7, 0.25, 1000.0, 1500.0, 1),
 }
 # cells of one value each, and their views: the ends of the detector that the image overhangs
 CELLS = {"overhang": ((0, 1), (2, 0), (20, 2), (39, 4)), "overhang_arc": ((0, 1), (2, 0), (20, 2), (39, 4)),
-         "fine_cells": ((70, 0), (101, 2), (130, 4))}
+         "far_overhang": ((0, 1), (39, 4)), "fine_cells": ((70, 0), (101, 2), (130, 4))}
 BETAS = np.array([0.05, 0.2, np.pi / 4, 0.9, 1.1])  # a short arc, so that pixels stay unseen
 
 
@@ -80,3 +82,35 @@ def test_back_keeps_values_that_are_not_finite_in_their_pixels(name, kind, dt, b
             assert not (must & ~bad).any(), (value, cell, view)
             assert not (bad & ~may).any(), (value, cell, view, int((bad & ~may).sum()))
             np.testing.assert_array_equal(got[~may], want[~may])
+
+
+@pytest.mark.parametrize("det", [1, 0])
+@pytest.mark.parametrize("kind", ["dd", "tf"])
+def test_back_of_images_far_beyond_the_detector_vs_fp64_oracle(kind, det):
+    """The form that passes over views, an odd number of them, alone and in a batch with a slice
+    that would not take it: relative L2 <= 1e-5, the repository's FP32 gate, or three times the
+    FP32 oracle's own distance where that is larger, as in the other parity tests."""
+    from conftest import rel_l2
+    from oracle import oracle as O
+    from ctsim_amd.batch2 import Batch2
+    from ctsim_amd.device import DeviceArray
+    from ctsim_amd.projector import Projector
+    rng = np.random.default_rng(5)
+    betas = rng.uniform(0, 2 * np.pi, 27)
+    far = O.G2(259, 257, 1.1, 1.0, 2.0, -1.0, 41, 1.3, 3.0, 1000.0, 0.0, 1500.0, betas, det)
+    near = O.G2(70, 61, 0.8, 0.8, 0.0, 0.0, 130, 1.0, 0.25, 1000.0, 0.0, 1500.0, betas[:6], det)
+    sinos = [(0.2 + rng.uniform(0, 1, (g.nu, g.nviews))).astype(np.float32) for g in (far, near)]
+    wants = [O.fbct(f"back,{kind}", g, s, prec=64) for g, s in zip((far, near), sinos)]
+    tols = [max(1e-5, 3 * rel_l2(O.fbct(f"back,{kind}", g, s), w)) for g, s, w in zip((far, near), sinos, wants)]
+    P = Projector(geometry_from_g2(far))
+    out = DeviceArray(P.n_img, "f32")
+    P.back(P.upload_sino(sinos[0]), out, f"back,{kind}")
+    assert rel_l2(P.download_volume(out), wants[0]) <= tols[0]
+    B = Batch2([geometry_from_g2(near), geometry_from_g2(far)])
+    img = DeviceArray(B.img_elems, "f32")
+    flat = np.concatenate([s.ravel(order="F") for s in sinos[::-1]])
+    for split in (1, 2, 4):
+        B.set_schedule(1, split)
+        B.back(DeviceArray.from_numpy(flat, "f32"), img, f"back,{kind}")
+        for got, want, tol in zip(B.unpack_images(img.to_numpy()), wants[::-1], tols[::-1]):
+            assert rel_l2(got, want) <= tol, (split, rel_l2(got, want))
