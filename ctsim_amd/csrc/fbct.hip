@@ -43,6 +43,8 @@ enum Foot2 { F2_DD = 0, F2_TF = 1 };
 // amp = dx / max(|cos|, |sin|) / 10 = dx hypot(X, Y) / max(|X|, |Y|) / 10 with (X, Y) the
 // pixel relative to the source.
 //
+// EACH: fan_lines_each, for tiles that meet a value that is not finite.
+//
 // Each wave stages kFanWords words of amp * pixel at a time (16 lines of 100 pixels, or 8 of
 // 196) in LDS, zero outside the image: amp is formed once per pixel, and image columns are
 // read 8 or 16 neighbours at a time instead of one word per image row.  Tiles whose rays
@@ -119,8 +121,57 @@ __device__ __forceinline__ float fan_lines(const FanLane& L, const float* buf, i
     return acc;
 }
 
+// the same lines pixel by pixel, without those that the cell does not overlap: the telescoped sum
+// takes a value that is not finite to the cells beside it (0 Inf, Inf - Inf).  K = 4 covers every
+// tile.
+template <int FOOT, bool ARC>
+__device__ __forceinline__ float fan_lines_each(const FanLane& L, const float* buf, int P, int jb, int m0, int nl, float wmaj,
+                                                float dmaj, float inv3) {
+    constexpr int K = 4;
+    float acc = 0.f;
+    const float ah = FOOT == F2_TF ? fabsf(L.h) : 0.f;
+    const float dden = ARC ? fmaf(L.kk, L.dt, L.dd) : L.dd;
+    const float gh = FOOT == F2_TF ? L.G * L.h : 0.f;
+#pragma unroll 1
+    for (int i = 0; i < nl; ++i) {
+        const float maj = (float(m0 + i) + wmaj) * dmaj;
+        const float xi = fmaf(maj, L.rho, L.cst);
+        const float jf = floorf(xi - ah);
+        const float* pq = buf + (i * P + (int)__builtin_amdgcn_fmed3f(jf - float(jb), 0.f, float(P - K)));
+        float den = fmaf(jf, dden, fmaf(maj, L.cmaj, L.dconst));
+        if constexpr (ARC) den = fmaf(L.kk, fmaf(maj, L.tmaj, L.tconst), den);
+        float c0 = 0.f, a0 = 0.f;  // part of the cell before the pixel's first edge, and that edge's start
+#pragma unroll 1
+        for (int k = 1; k <= K; ++k) {
+            const float dk = fmaf(float(k), dden, den), num = ((jf - xi) + float(k)) * L.G;
+            auto edge = [&](float nu_, float de_) {
+                float f = nu_ * frcp(de_);
+                if constexpr (ARC) f = fmaf(f * f, -inv3 * f, f);
+                return f;
+            };
+            float c, a, b;
+            if constexpr (FOOT == F2_DD) {
+                a = b = edge(num, dk);
+                c = clamp01(a);
+            } else {
+                const float e0 = edge(num - gh, dk + L.hd), e1 = edge(num + gh, dk - L.hd);
+                a = fminf(e0, e1);
+                b = fmaxf(e0, e1);
+                const float i2 = 0.5f * frcp(fmaxf(b - a, 1.0e-20f));
+                const float z1 = __builtin_amdgcn_fmed3f(1.f, a, b) - a, z0 = __builtin_amdgcn_fmed3f(0.f, a, b) - a;
+                c = 1.f - ((z1 - z0) * (z1 + z0) * i2 + fmaxf(1.f - b, 0.f) - fmaxf(-b, 0.f));
+            }
+            if (k == K) c = b = 1.f;
+            if (a0 < 1.f && b > 0.f) acc = fmaf(c - c0, pq[k - 1], acc);
+            c0 = c;
+            a0 = a;
+        }
+    }
+    return acc;
+}
+
 // the walks of one tile over share `share` of `nshares` of the lines
-template <class Tin, int FOOT, bool ARC>
+template <class Tin, int FOOT, bool ARC, bool EACH>
 __device__ __forceinline__ float fan_tile(const Geom<float>& g, const View<float>& v, int ut, const Tin* __restrict__ img,
                                           int exhaustive, int share, int nshares, float* buf) {
     const int lane = lane_id();
@@ -179,7 +230,7 @@ __device__ __forceinline__ float fan_tile(const Geom<float>& g, const View<float
         const float wpx = fmaf(fmaxf(fmaxf(width(0, 1, y0), width(0, 1, y1)),
                                      fmaxf(width(kW2 - 2, kW2 - 1, y0), width(kW2 - 2, kW2 - 1, y1))),
                                1.05f, 2.f * hm + 0.01f);
-        const int K = uni(wpx <= 1.f ? 2 : wpx <= 2.f ? 3 : 4);
+        const int K = uni(EACH ? 4 : wpx <= 1.f ? 2 : wpx <= 2.f ? 3 : 4);
         // staged width of one line, its drift from line to line, and the lines per chunk
         const float span = fmaxf(width(0, kW2 - 1, y0), width(0, kW2 - 1, y1)) + 2.f * hm + float(K + 4);
         const float drift = fmaxf(fabsf(rho0), fabsf(rho1)) * dmaj;
@@ -275,7 +326,8 @@ __device__ __forceinline__ float fan_tile(const Geom<float>& g, const View<float
             if (gen) fill(std::true_type{});
             else fill(std::false_type{});
             __builtin_amdgcn_wave_barrier();
-            if (K == 2) acc += fan_lines<FOOT, ARC, 2>(L, buf, P, jb, m0, nl, wmaj, dmaj, inv3);
+            if constexpr (EACH) acc += fan_lines_each<FOOT, ARC>(L, buf, P, jb, m0, nl, wmaj, dmaj, inv3);
+            else if (K == 2) acc += fan_lines<FOOT, ARC, 2>(L, buf, P, jb, m0, nl, wmaj, dmaj, inv3);
             else if (K == 3) acc += fan_lines<FOOT, ARC, 3>(L, buf, P, jb, m0, nl, wmaj, dmaj, inv3);
             else acc += fan_lines<FOOT, ARC, 4>(L, buf, P, jb, m0, nl, wmaj, dmaj, inv3);
             __builtin_amdgcn_wave_barrier();
@@ -440,7 +492,15 @@ __device__ __forceinline__ T fbct_proj_item(const Geom<T>& g, const View<T>& v, 
         return fbct_proj_acc<Tin, T, FOOT>(g, v, ut, img, exhaustive, share, nshares);
     } else {
         __shared__ __align__(16) float buf[4][kFanWords];
-        return fan_tile<Tin, FOOT, FORM == 2>(g, v, ut, img, exhaustive, share, nshares, buf[threadIdx.x / kW2]);
+        float* const b = buf[threadIdx.x / kW2];
+        const float acc = fan_tile<Tin, FOOT, FORM == 2, false>(g, v, ut, img, exhaustive, share, nshares, b);
+        // a value that is not finite stays with the cells that it weighs on: the sums of those that
+        // came out not finite again, pixel by pixel.  (In the arc kernels whose waves share a tile
+        // the second copy of the walk costs one to three spilled registers, 0 to 9% for images of
+        // up to 64^2 pixels.)
+        if (__builtin_expect(!__any(!__builtin_isfinite(acc)), 1)) return acc;
+        const float each = fan_tile<Tin, FOOT, FORM == 2, true>(g, v, ut, img, exhaustive, share, nshares, b);
+        return __builtin_isfinite(acc) ? acc : each;
     }
 }
 

@@ -114,3 +114,51 @@ def test_back_of_images_far_beyond_the_detector_vs_fp64_oracle(kind, det):
         B.back(DeviceArray.from_numpy(flat, "f32"), img, f"back,{kind}")
         for got, want, tol in zip(B.unpack_images(img.to_numpy()), wants[::-1], tols[::-1]):
             assert rel_l2(got, want) <= tol, (split, rel_l2(got, want))
+
+
+def _proj(name, kind, img, dt, batch):
+    from ctsim_amd.batch2 import Batch2
+    from ctsim_amd.device import DeviceArray
+    from ctsim_amd.projector import Projector
+    geom = geometry_from_g2(_fan(name))
+    if not batch:
+        P = Projector(geom)
+        out = DeviceArray(P.n_sino(), "f32")
+        P.proj(P.upload_volume(img, dt), out, f"proj,{kind}")
+        return P.download_sino(out)
+    B = Batch2([geom, geom])
+    out = DeviceArray(B.sino_elems, "f32")
+    B.proj(DeviceArray.from_numpy(B.pack_images([img, img]), dt), out, f"proj,{kind}")
+    a, b = B.unpack_sinos(out.to_numpy())
+    np.testing.assert_array_equal(a, b)
+    return a
+
+
+@pytest.mark.parametrize("batch", [False, True])
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("kind", ["dd", "tf"])
+@pytest.mark.parametrize("name", [n for n in FANS if n != "far_overhang"])
+def test_proj_keeps_values_that_are_not_finite_in_their_cells(name, kind, dt, batch):
+    """the other cells keep their values to the repository's FP32 gate, 1e-5 of the largest (the
+    same products may be added in another order)"""
+    from oracle import oracle as O
+    rng = np.random.default_rng(4)
+    nx, ny = FANS[name][0]
+    clean = (0.2 + rng.uniform(0, 1, (nx, ny))).astype(np.float32)
+    want = _proj(name, kind, clean, dt, batch)
+    assert np.isfinite(want).all()
+    for value in (np.nan, np.inf):
+        for ix, iy in ((nx // 2 - 4, ny // 2), (nx // 2, 0), (nx // 2 - 2, ny - 1)):
+            only = np.zeros_like(clean)
+            only[ix, iy] = 1
+            low, weight, high = (O.fbct(f"proj,{kind}", _fan(name, s), only, prec=64) for s in SHIFTS)
+            must = weight > 1e-6 * weight.max()
+            may = (low != 0) | (weight != 0) | (high != 0)
+            assert must.any()
+            img = clean.copy()
+            img[ix, iy] = value
+            got = _proj(name, kind, img, dt, batch)
+            bad = ~np.isfinite(got)
+            assert not (must & ~bad).any(), (value, ix, iy)
+            assert not (bad & ~may).any(), (value, ix, iy, int((bad & ~may).sum()))
+            np.testing.assert_allclose(got[~may], want[~may], rtol=0, atol=1e-5 * want.max())
