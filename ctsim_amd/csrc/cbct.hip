@@ -1832,15 +1832,17 @@ __global__ __launch_bounds__(kBlock) void cbct_back_kernel(Geom<T> g, const View
 //  * a lane loads four rows of each footprint cell at once (8 or 16 bytes; one load per cell and
 //    64 rows of four columns, where the one-column form takes one per cell and column), combines
 //    them and writes them to its column's row buffer, words of rows past the detector as zeros;
-//  * the next view's first rows load while this one is gathered;
+//  * views that miss the four columns are passed over, and the next view's first rows load while
+//    this one is gathered;
 //  * lane l % 16 owns voxels l % 16 + 16 i of its column, all parameters in vector registers.
 //
-// Latency bounds it, as it does the one-column form (which ran no faster with its footprint
-// arithmetic cut by a fifth): three blocks of four waves per CU where the column's 32 voxels per
-// lane need the registers (at four they spill: 512-slice columns 3.95 ms against 2.16), else
-// four (six spill FP32: 62.5 ms against 51.9 below).  Against the one-column form: SF of 512^2 x
-// 128 from a subset of 41 BF16 views 0.93 -> 0.80 ms; DD of 512^2 x 256 from 720 FP32 views
-// 82.6 -> 51.9 ms; DD of 256^2 x 512 from 60 views 3.09 -> 2.16 ms.
+// Three blocks of four waves per CU where the column's 32 voxels per lane need the registers
+// (164 of 168), else four (116 of 128 at 16 voxels per lane; nothing spills).  Against the
+// one-column form: SF of 512^2 x 128 from a subset of 41 BF16 views 0.93 -> 0.72 ms; DD of 512^2 x
+// 256 from 720 FP32 views 82.6 -> 49.5 ms; DD of 256^2 x 512 from 60 views of 400 rows 2.43 ->
+// 1.43 ms.  (A loop over every view of a batch, seen or not, kept 12 more registers and took 0.80,
+// 52.2 and 1.65 ms, and 1.6 times the one-column form's time where few views see a column: 128^2 x
+// 64 on a detector of a tenth of its shadow, 42 us against 26.)
 // ---------------------------------------------------------------------------------
 constexpr int kQuadRows = 768;  // four row buffers per wave within 64 KB of LDS per block
 constexpr int kQuadViews = 16, kQuadRec = 14;  // views per batch, words per record
@@ -1919,7 +1921,8 @@ __global__ __launch_bounds__(kBlock, NZ >= 32 ? 3 : 4) void cbct_back_quad_kerne
         for (int b0 = 0; b0 < nviews; b0 += kQuadViews) {
             const int nb = min(kQuadViews, nviews - b0);
             // footprint of view b0 + l16 on this lane's column; columns that the view misses get
-            // zero weights and no cells
+            // zero weights and no cells, and views that miss all four are passed over (todo)
+            unsigned todo;
             {
                 float4* rec = recs + l16 * 4 + l4;
                 bool ok = active && l16 < nb;
@@ -1953,7 +1956,10 @@ __global__ __launch_bounds__(kBlock, NZ >= 32 ? 3 : 4) void cbct_back_quad_kerne
                 rec[64] = rw;
                 rec[128] = rx;
                 recx[l16 * 4 + l4] = make_int2(voff, rows);
+                const unsigned long long m = __ballot(ok);
+                todo = (unsigned)(m | m >> 16 | m >> 32 | m >> 48) & 0xffffu;
             }
+            if (todo == 0) continue;
             __builtin_amdgcn_wave_barrier();
             const auto rs = buf_rsrc(proj + (size_t)b0 * view_elems, (int)((unsigned)nb * (unsigned)view_elems * (unsigned)sizeof(Tin)));
             Rows4<Tin> pre[4];
@@ -1976,19 +1982,16 @@ __global__ __launch_bounds__(kBlock, NZ >= 32 ? 3 : 4) void cbct_back_quad_kerne
                         last = max(last, b);
                     }
                 }
-                if (last < 0) return;
                 first >>= 6;
                 last = min((last + kRowPad) >> 6, (g.nv - 1) >> 6);
                 load4((unsigned)rc.x + (unsigned)((64 * first + row0) * (int)sizeof(Tin)), rc.y >> 20, pre);
             };
-            begin(0);
-            for (int k = 0; k < nb; ++k) {
+            begin(__builtin_ctz(todo));
+            while (todo != 0) {
+                const int k = __builtin_ctz(todo);
+                todo &= todo - 1;
                 const float4* rec = recs + k * 4 + l4;
                 const int c0 = first, c1 = last;
-                if (c1 < 0) {
-                    if (k + 1 < nb) begin(k + 1);
-                    continue;
-                }
                 const float4 w = rec[64];
                 const int2 rc = recx[k * 4 + l4];
                 const int cells = rc.y >> 20;
@@ -2033,7 +2036,7 @@ __global__ __launch_bounds__(kBlock, NZ >= 32 ? 3 : 4) void cbct_back_quad_kerne
                     *(float4*)(sw + 4 + 64 * c + row0) = o;
                 }
                 __builtin_amdgcn_wave_barrier();
-                if (k + 1 < nb) begin(k + 1);
+                if (todo != 0) begin(__builtin_ctz(todo));
                 const float4 ra = rec[0];
                 const T zinc = ra.x, r2 = ra.z;
                 // the group's class: rows that its thickest voxels meet
@@ -2703,23 +2706,33 @@ static void launch_back_dd_tf(unsigned blocks, hipStream_t st, const Geom<T>& g,
 
 // whether the four-column form takes a backprojection: FP32, voxels of at most three rows at
 // the nearest column, footprints of at most kQuadCells cells, rows addressed in whole words,
-// and enough columns that a quarter of the waves still fills the chip:
-// below that the one-column form's larger number of waves wins (64 slices: 64^2 columns 45 us
-// against 69, 112^2 98 against 101, 256^2 345 against 292; 256 slices: 64^2 146 against 167,
-// 80^2 245 against 211, 128^2 421 against 268).  On detectors of at most 64 rows the one-column
-// form keeps a whole column's rows in one pass and its taller columns win unless the image is
-// large (106 x 102 x 142 from 58 rows FP16 124 us against 147, 252 x 197 x 80 FP32 1007 against
-// 1081, 500 x 350 x 143 BF16 744 against 759; but 512^2 x 128 BF16 934 against 803)
+// and enough columns that a quarter of the waves still fills the chip; below that the one-column
+// form's larger number of waves wins.  Microseconds, one column / four, FP32 unless said:
+//  * up to 64 slices, SF, 64 rows, 41 views: 64^2 26 / 34, 80^2 39 / 44, 96^2 45 / 44, 112^2
+//    63 / 52, 128^2 67 / 51, 256^2 228 / 158;
+//  * taller, over 64 rows, DD, 60 views: 256 slices 64^2 114 / 112, 72^2 155 / 155, 80^2 190 / 157,
+//    128^2 323 / 201; 100 slices 64^2 84 / 68, 80^2 141 / 87;
+//  * taller, at most 64 rows (the one-column form keeps a whole column's rows in one pass), SF, 41
+//    views: 80 slices BF16 200^2 171 / 148, 256^2 238 / 193, 320^2 369 / 289, 512^2 927 / 710,
+//    FP16 alike, and 128 slices alike; FP32 stays with the one-column form, though 128 slices from
+//    200^2 columns on now gain too (169 / 153, 256^2 238 / 201, 512^2 912 / 742); 143 slices 256^2
+//    FP32 298 / 318, BF16 306 / 313, 512^2 1133 / 1215 and 1187 / 1183.
+// Where the detector reaches only part of the image's shadow, the waves of unseen columns end
+// early and more columns are needed.  128^2 on a detector of 0.6, 0.3 and 0.1 of it: 64 slices and
+// rows 60 / 50, 38 / 40 and 26 / 35, 100 of each 98 / 73, 60 / 58 and 41 / 51; 200^2 x 300 at 0.1
+// 186 / 142.
 template <class Tin, class T, int NZL>
 static bool quad_ok(const Geom<T>& g, const void* proj) {
     if constexpr (sizeof(T) != 4) return false;
     if (g.nv > kQuadRows) return false;
-    const long long cols = (long long)g.nx * g.ny;
-    if (NZL == 1 ? cols < 16384 : g.nv > kWave ? cols < 6400 : NZL > 2 || sizeof(Tin) != 2 || cols < 65536) return false;
-    if ((g.nv * sizeof(Tin)) % 4 != 0 || (uintptr_t)proj % 4 != 0) return false;
     const double hx = std::max(std::fabs((double)g.wx), std::fabs((double)g.wx + g.nx - 1)) * std::fabs((double)g.dx);
     const double hy = std::max(std::fabs((double)g.wy), std::fabs((double)g.wy + g.ny - 1)) * std::fabs((double)g.dy);
     const double R = std::sqrt(hx * hx + hy * hy);
+    // how far the detector reaches, of the image's shadow
+    const double reach = std::max(std::fabs((double)g.wu), std::fabs((double)g.wu + g.nu - 1)) * g.sad;
+    const double cols = (double)g.nx * g.ny, seen = cols * std::min(1.0, 2.5 * reach / (R * std::fabs((double)g.sdd_du)));
+    if (NZL == 1 ? seen < 16384 : g.nv > kWave ? seen < 6400 : NZL > 2 || sizeof(Tin) != 2 || cols < 65536) return false;
+    if ((g.nv * sizeof(Tin)) % 4 != 0 || (uintptr_t)proj % 4 != 0) return false;
     if (!(g.zk > 0 && g.sad > R * 1.001 && g.zk / (g.sad - R) * 1.001 <= 3.0)) return false;
     // footprint width in cells: the pixel's angle from the source, times the cells per radian at
     // the edge of the image on a flat detector; a width of w meets at most w + 2 cells
