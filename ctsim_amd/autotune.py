@@ -1,7 +1,8 @@
 """Schedule cache of the 3D autotuner (ctsim_plan_autotune).
 
 A tuned schedule depends on the operator, the geometry, the view selection, the storage
-dtypes and the GPU, not on the data, so it is measured once and kept in a JSON file
+dtypes, the GPU and the kernels that its codes stand for, not on the data, so it is measured
+once for a built library and kept in a JSON file
 (``$CTSIM_SCHEDULE_CACHE``, default ``~/.cache/ctsim_amd/schedules.json``):
 
     from ctsim_amd.autotune import tuned
@@ -12,10 +13,12 @@ block per detector column (geom/dd_cuda/cbct_dd_proj.c:441-442).
 """
 from __future__ import annotations
 
+import functools
 import hashlib
 import json
 import os
 
+from . import _lib
 from .projector import Projector
 from .device import DeviceArray
 
@@ -33,11 +36,19 @@ def _device_name() -> str:
         return "gpu"
 
 
+@functools.lru_cache(maxsize=None)
+def _kernels(path: str) -> str:
+    """What the schedule codes stand for: the library that was built.  A code timed with other
+    kernels may be the slower one here, and its times are not these kernels'."""
+    with open(path, "rb") as f:
+        return hashlib.sha1(f.read()).hexdigest()[:12]
+
+
 def schedule_key(P: Projector, op: str, view0: int, vstep: int, nsub: int, in_dt: int, out_dt: int) -> str:
     g = P.geom
     fields = [op, g.reconSize, g.reconSpacing, g.reconOffset, g.detSize, g.detSpacing, g.detOffset, g.SAD, g.SDD,
               g.flatPanel, view0, vstep, nsub, in_dt, out_dt, P.compute, _device_name(),
-              hashlib.sha1(g.betas.tobytes()).hexdigest()[:12]]
+              _kernels(_lib.LIB_PATH), hashlib.sha1(g.betas.tobytes()).hexdigest()[:12]]
     return hashlib.sha1(repr(fields).encode()).hexdigest()[:20]
 
 
