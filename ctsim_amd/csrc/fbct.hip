@@ -521,7 +521,9 @@ __global__ __launch_bounds__(256, FORM ? kFanWaves : 1) void fbct_proj_kernel(Ge
         // the view in registers (a wave-uniform index: scalar loads, once per item), so that
         // the walk's LDS atomics and barriers do not make the compiler reload it every batch
         const View<T> vw = views[(size_t)uni(b) * vstride];
-        acc = fbct_proj_item<Tin, T, FOOT, FORM>(g, vw, uni(ut), img, exhaustive, wv % S, S);
+        // (the tile in a scalar register is for the line walk: it cost the candidate form 1 to 3%,
+        // SF of 512^2 at 0.5 mm on 1024 bins of 0.8 mm, 984 views, 2410 against 2447 us)
+        acc = fbct_proj_item<Tin, T, FOOT, FORM>(g, vw, FORM ? uni(ut) : ut, img, exhaustive, wv % S, S);
     }
     if (S > 1) {
         part[wv][lane] = acc;
