@@ -446,9 +446,9 @@ int ctsim_plan_autotune(ctsim_plan* p, const char* op, int32_t view0, int32_t vs
         return fail(CTSIM_EINVAL, "Error: the 3D autotuner takes proj,dd proj,tf back,dd back,tf back,pd back,hpd.");
     if (d_in == d_out) return fail(CTSIM_EINVAL, "Error: the tuning output must not alias the input.");
     if (reps < 1) reps = 1;
-    // the forward schedules (form | split << 2): automatic, LDS ring with whole and with shared
-    // items, register pipeline with whole and with shared items, the ring with two row chunks
-    // per item (whole items); the backward column orders
+    // the forward schedules (form | split << 2): automatic, matrix or LDS-ring form with whole and
+    // with shared items, register pipeline with whole and with shared items, matrix or ring form
+    // with two row chunks per item (whole items); the backward column orders
     // (DD / SF) or the FDK backprojection's staged and direct forms (pd / hpd), each keeping
     // the other bit of the current schedule
     static const int kProj[6] = {0, 1 | (1 << 2), 1 | (2 << 2), 2 | (1 << 2), 2 | (2 << 2), 3 | (1 << 2)};

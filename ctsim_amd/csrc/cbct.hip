@@ -918,7 +918,8 @@ __global__ __launch_bounds__(WPB * kWave, kRingWaves) void cbct_proj_ring_kernel
 
 // ---------------------------------------------------------------------------------
 // Forward projection, matrix form (FP32 volumes whose voxels are 1/4 to 14 rows thick on the
-// detector everywhere).  The same work items, strips, footprints and row gathers as the ring
+// detector everywhere and of whose columns an item's rows need at most 128 voxels: mat_voxels).
+// The same work items, strips, footprints and row gathers as the ring
 // form; what differs is what happens to a surviving column's 64 RPL row sums.  A tile is
 //     p[cell, row] = sum over columns of w[cell, column] q[column, row],
 // a product whose inner dimension is the strip's columns, so four columns at a time go to the
@@ -938,10 +939,12 @@ __global__ __launch_bounds__(WPB * kWave, kRingWaves) void cbct_proj_ring_kernel
 //    whose tile ends up with one walks its item again and adds each footprint's own cells only;
 //  * a footprint of more than four tile cells takes a record for every four of them.
 //
-// 45 vector and 6 scalar instructions per column and item against the ring form's 57 and 48
+// 44 vector and 5 scalar instructions per column and item against the ring form's 57 and 48
 // (SF, 41 views of 1024 x 64 over 512^2 x 128: 1.47 -> 0.90 ms; 720 views of 1024 x 384 over
-// 512^2 x 256, two row chunks per item: 112 -> 58 ms).  It now waits on memory as much as on
-// issue: each view reads the volume once from beyond L2.
+// 512^2 x 256, two row chunks per item: 112 -> 58.6 ms).  In the first its waves spend a third of
+// their cycles waiting for issue and a third on counters (each view reads the volume once from
+// beyond L2), and a third of the LDS cycles are bank conflicts; with two row chunks it is 43% for
+// issue and 28% on counters, no conflicts, and 11 to 19 registers spilled.
 // ---------------------------------------------------------------------------------
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kRecWords = 12;           // one column's record
@@ -1836,8 +1839,11 @@ __global__ __launch_bounds__(kBlock) void cbct_back_kernel(Geom<T> g, const View
 //    this one is gathered;
 //  * lane l % 16 owns voxels l % 16 + 16 i of its column, all parameters in vector registers.
 //
-// Three blocks of four waves per CU where the column's 32 voxels per lane need the registers
-// (164 of 168), else four (116 of 128 at 16 voxels per lane; nothing spills).  Against the
+// Bound by instruction issue: on the subset below its waves spend 46% of their cycles waiting for
+// issue and 19% on counters; with FP32 views and 16 voxels per lane 20% and 34%, and a third of the
+// LDS cycles are bank conflicts.  Three blocks of four waves per CU where the column's 32 voxels
+// per lane need the registers (164 of 168), else four (116 of 128 at 16 voxels per lane; nothing
+// spills).  Against the
 // one-column form: SF of 512^2 x 128 from a subset of 41 BF16 views 0.93 -> 0.72 ms; DD of 512^2 x
 // 256 from 720 FP32 views 82.6 -> 49.5 ms; DD of 256^2 x 512 from 60 views of 400 rows 2.43 ->
 // 1.43 ms.  (A loop over every view of a batch, seen or not, kept 12 more registers and took 0.80,
@@ -2512,7 +2518,9 @@ constexpr int kHalfRing1 = 6, kHalfRing2 = 4;
 
 // voxels of a column that the matrix form stages for an item of `rows` detector rows, 0 where
 // it does not cover the geometry: a voxel's height on the detector is zk / d rows, d between
-// the nearest and the farthest column's distance; the volume is addressed with 32-bit offsets
+// the nearest and the farthest column's distance; the volume is addressed with 32-bit offsets.
+// At most 128 are staged: volumes of more than 128 slices are covered down to 0.52 rows per voxel
+// at the farthest column for items of 64 rows and 1.04 for items of 128, shorter ones to 1/4.
 static int mat_voxels(const Geom<float>& g, int rows) {
     const double hx = std::max(std::fabs((double)g.wx), std::fabs((double)g.wx + g.nx - 1)) * std::fabs((double)g.dx);
     const double hy = std::max(std::fabs((double)g.wy), std::fabs((double)g.wy + g.ny - 1)) * std::fabs((double)g.dy);
@@ -2545,8 +2553,9 @@ static void launch_proj(unsigned blocks, hipStream_t st, const Geom<T>& g, const
             return;
         }
     }
-    // the matrix form wherever it covers the geometry and the schedule does not ask for the
-    // register pipeline; RPL and the grid come from proj3_foot (form 3: two row chunks per item)
+    // the matrix form where it covers the geometry at the items' rows and the schedule does not
+    // ask for the register pipeline; RPL and the grid come from proj3_foot (form 3: two row chunks
+    // per item, which a geometry may be covered without and not with: those take the ring form)
     if constexpr (std::is_same<Tin, float>::value && std::is_same<T, float>::value) if (form != 2) {
         const int rows = form == 3 ? 2 * kWave : kWave, need = mat_voxels(g, rows);
         if (need > 0) {
@@ -2618,10 +2627,12 @@ static void launch_proj(unsigned blocks, hipStream_t st, const Geom<T>& g, const
 template <class Tin, class Tout, class T, int FOOT>
 static void proj3_foot(const Geom<T>& g, const View<T>* views, int vstride, int nviews, const void* vol,
                        const uint8_t* map, void* proj, int exhaustive, hipStream_t st) {
-    // form 3: eight-cell tiles of two 64-row chunks, one wave per item (FP32 volumes of at
-    // most 256 slices; other volumes take the automatic choice).  Automatic: taken for
-    // detectors over 64 rows whose items need no split (measured on the 720-view
-    // 512^2 x 256 pair at 1024 x 384: SF forward 146 -> 115 ms, DD 134 -> 102 ms)
+    // form 3: two 64-row chunks per item, one wave per item (FP32 volumes of at most 256 slices;
+    // other volumes take the automatic choice), in 16-cell tiles where the matrix form covers the
+    // geometry at 128 rows, else in the ring form's eight-cell ones.  Automatic: taken for
+    // detectors over 64 rows whose items need no split (the 720-view 512^2 x 256 pair at 1024 x
+    // 384 in the ring form: SF forward 146 -> 115 ms, DD 134 -> 102; in the matrix form's two
+    // chunks 58.6 and 54.7)
     constexpr bool fp32 = std::is_same<Tin, float>::value && std::is_same<T, float>::value;
     const int form = g.sched_proj & 3, ssplit0 = (g.sched_proj >> 2) & 3;
     const long long items1 = (long long)nviews * ((g.nu + kTU - 1) / kTU) * ((g.nv + kWave - 1) / kWave);

@@ -53,8 +53,9 @@ enum Foot2 { F2_DD = 0, F2_TF = 1 };
 //
 // Issue-bound: 47 vector instructions per (line, 64 cells) all told, against some 230 per 64
 // pixels of the candidate form below with its LDS min / max.  256^2, 360 views, 512 bins, DD:
-// 239 -> 86 us; 64 uneven FP16 slices: 18.4 -> 6.1 ms.  The distance from 64-bit results went
-// from 3.3e-6 to 2.0e-6 (no subtraction of large detector coordinates).
+// 239 -> 86 us (the pair's few waves wait for issue 41% of their cycles and on counters 31%); 64
+// uneven FP16 slices: 18.4 -> 6.1 ms (51% and 13%).  The distance of the pair from 64-bit results
+// went from 3.3e-6 to 2.4e-6 (no subtraction of large detector coordinates).
 // ---------------------------------------------------------------------------------
 constexpr int kFanWaves = 6;     // waves per SIMD the line-walk kernels are compiled for
 constexpr int kFanWords = 1600;  // staged words per wave: six 4-wave blocks fit a CU's LDS
@@ -549,9 +550,9 @@ __global__ __launch_bounds__(256, FORM ? kFanWaves : 1) void fbct_proj_kernel(Ge
 //   SF: cell k weighs C(k + 1) - C(k), C the trapezoid's running integral, the difference of
 //     its two ramps' integrals; two reciprocals per pixel where the per-cell form takes two
 //     per cell.
-// Bound by instruction issue: 96 -> 55 (DD) vector instructions per 64 pixel-views, with the
-// views through scalar loads.  256^2, 360 views, DD: 75 -> 43 us; 64 uneven FP16 slices:
-// 7.97 -> 4.37 ms.
+// Bound by instruction issue where there are waves enough: 98 -> 56 (DD) vector instructions per
+// 64 pixel-views, with the views through scalar loads.  64 uneven FP16 slices: 7.5 -> 4.3 ms;
+// 256^2, 360 views, DD: 75 -> 43 us (16 waves per CU, which wait on counters 42% of their cycles).
 // The cells are returned as loaded: the caller evaluates a second view's footprint before it
 // uses them.
 // EACH: only cells that the footprint reaches are read.  Without it (DD) those after its end weigh

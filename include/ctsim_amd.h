@@ -187,23 +187,24 @@ int ctsim_plan_destroy(ctsim_plan* plan);
 /* Launch schedules of a 3D plan (no counterpart in the reference, whose CUDA path uses
  * fixed 16 x 16 blocks, geom/dd_cuda/cbct_dd_proj.c:441-442).  proj_sched = form | split << 2:
  * form 0 automatic, 1 the matrix forward kernel (FP32 volumes whose voxels are 1/4 to
- * 14 detector rows thick) or the LDS-ring one (other FP32 volumes of at most 256 slices, FP16
- * volumes of an even number of at most 256), 2 register-pipeline forward kernel, 3 the same
- * with two 64-row chunks per item (FP32 volumes in the matrix kernel's range, or of at most 256
- * slices; one wave per item; others take the automatic form); split 0
+ * 14 detector rows thick, of at most 128 slices or of voxels of at least about half a row) or the
+ * LDS-ring one (other FP32 volumes of at most 256 slices, FP16 volumes of an even number of at
+ * most 256), 2 register-pipeline forward kernel, 3 as 1 with two 64-row chunks per item (FP32
+ * volumes of at most 256 slices, the matrix kernel there for at most 128 slices or voxels of at
+ * least about one row; one wave per item; others take the automatic form); split 0
  * automatic (a block's waves share a work item below 16384 items), 1 one wave per item,
  * 2 shared items.  back_sched bit 0 (DD / SF backprojection): 0 consecutive image columns, 1
- * 2 x 2 column patches in 32 x 32 super-tiles (either way the same terms in the same order); bit 1 (FDK pd / hpd, FP32 plans): 0 the LDS-staged form (detectors of at
- * most 1024 rows; taller ones take the direct form), 1 the direct form.  A new plan has
- * (0, 1).  Every schedule is deterministic; the forward forms and splits, and the two FDK
+ * 2 x 2 column patches in 32 x 32 super-tiles (either way the same terms in the same order);
+ * bit 1 (FDK pd / hpd, FP32 plans): 0 the LDS-staged form (detectors of at most 1024 rows; taller
+ * ones take the direct form), 1 the direct form.  A new plan has (0, 1).  Every schedule is deterministic; the forward forms and splits, and the two FDK
  * forms, add terms in different orders, so their results agree to FP32 rounding, not bit
  * for bit. */
 int ctsim_plan_set_schedule(ctsim_plan* plan, int32_t proj_sched, int32_t back_sched);
 int ctsim_plan_get_schedule(const ctsim_plan* plan, int32_t* proj_sched, int32_t* back_sched);
 
 /* The project's autotuner for 3D plans: times every forward schedule (op proj,dd or
- * proj,tf: automatic, ring whole, ring shared, register whole, register shared, ring with two
- * row chunks), every
+ * proj,tf: automatic, matrix or ring whole, the same shared, register whole, register shared,
+ * matrix or ring with two row chunks), every
  * backprojector column order (back,dd or back,tf) or both FDK forms (back,pd or back,hpd)
  * on the caller's view selection and
  * buffers with HIP events on the stream (one warm-up, then reps timed launches each),
@@ -264,7 +265,10 @@ int ctsim_zxy_to_xyz(const void* d_src, int32_t src_dtype, void* d_dst, int32_t 
  * Batched uneven 2D slices: nslices independent fan-beam slices, each with its own
  * geometry and views, projected (or backprojected) in one launch.  Images and
  * sinograms of all slices are packed back to back in d_img / d_sino in slice order
- * ([nx ny] and [nu nviews] each).
+ * ([nx ny] and [nu nviews] each).  One kernel serves all slices of a launch: the FP32 forward's
+ * line walk needs every slice in its range (the source well outside the image, detector cells of
+ * at most three pixels) and detectors of one type; a single slice beyond that sends all of them
+ * to the slower candidate form (64 slices: 18.2 ms against 6.1).
  * ---------------------------------------------------------------------------- */
 typedef struct ctsim_batch2 ctsim_batch2;
 int ctsim_batch2_create(ctsim_batch2** batch, int32_t nslices, const ctsim_geom* geoms, const int32_t* nviews,
